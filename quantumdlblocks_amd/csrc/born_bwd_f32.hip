@@ -1,18 +1,33 @@
-// Backward kernel instantiations for fp32 inputs.
+// Backward kernel instantiations for fp32 inputs (Born; purified up to D = 128).
 #include "born_bwd.h"
+#include "born_f32.h"
 #include "born_launch.h"
+#include "purified_dispatch.h"
 
 namespace qdl {
 
 hipError_t bwd_launch_f32(const BwdArgs& a, hipStream_t s) {
+    if (a.D <= kF32MaxD) {
+        const hipError_t e = launch_f32_bwd<false>(a, s);
+        return e != hipSuccess ? e : launch_bwd_common_post(a, s);
+    }
     const int dp = padded_head_dim(a.D);
     const int mode = mask_mode(a.is_causal, a.window, a.doc);
 #define QDL_MODE_BODY(M) return launch_bwd32<DPV, M>(a, s);
 #define QDL_DP_BODY(D_) { constexpr int DPV = D_; QDL_SWITCH_MODE(mode, QDL_MODE_BODY) }
-    QDL_SWITCH_DP(dp, QDL_DP_BODY)
+    QDL_SWITCH_DP_WIDE(dp, QDL_DP_BODY)
 #undef QDL_DP_BODY
 #undef QDL_MODE_BODY
     return hipErrorInvalidValue;
+}
+
+hipError_t purified_bwd_f32_launch(const PurArgs& a, hipStream_t s) {
+    const hipError_t e = launch_f32_bwd<true>(a, s);
+    if (e != hipSuccess) return e;
+    const int n_scale = a.per_head_scale ? a.H : 1, n_tau = a.per_head_tau ? a.H : 1;
+    hipLaunchKernelGGL(purified_param_reduce_kernel<0>, dim3((unsigned)(n_scale + n_tau)), dim3(256), 0, s, a,
+                       f32_groups(a.B, a.H, a.T), n_scale);
+    return hipGetLastError();
 }
 
 }  // namespace qdl

@@ -1,18 +1,23 @@
-// Forward kernel instantiations for fp32 inputs.
+// Forward kernel instantiations for fp32 inputs (Born; purified up to D = 128).
+#include "born_f32.h"
 #include "born_fwd.h"
 #include "born_launch.h"
+#include "purified_dispatch.h"
 
 namespace qdl {
 
 hipError_t fwd_launch_f32(const FwdArgs& a, hipStream_t s) {
+    if (a.D <= kF32MaxD) return launch_f32_fwd<false>(a, s);
     const int dp = padded_head_dim(a.D);
     const int mode = mask_mode(a.is_causal, a.window, a.doc);
 #define QDL_MODE_BODY(M) return launch_fwd32<DPV, M>(a, s);
 #define QDL_DP_BODY(D_) { constexpr int DPV = D_; QDL_SWITCH_MODE(mode, QDL_MODE_BODY) }
-    QDL_SWITCH_DP(dp, QDL_DP_BODY)
+    QDL_SWITCH_DP_WIDE(dp, QDL_DP_BODY)
 #undef QDL_DP_BODY
 #undef QDL_MODE_BODY
     return hipErrorInvalidValue;
 }
+
+hipError_t purified_fwd_f32_launch(const PurArgs& a, hipStream_t s) { return launch_f32_fwd<true>(a, s); }
 
 }  // namespace qdl

@@ -41,6 +41,16 @@ hipError_t bwd_launch_f32(const BwdArgs& a, hipStream_t s);
         default: return hipErrorInvalidValue;         \
     }
 
+// The padded head dims above 128 (the staged fp32 kernels).
+#define QDL_SWITCH_DP_WIDE(dp, BODY)                  \
+    switch (dp) {                                     \
+        case 160: { BODY(160); } break;               \
+        case 192: { BODY(192); } break;               \
+        case 224: { BODY(224); } break;               \
+        case 256: { BODY(256); } break;               \
+        default: return hipErrorInvalidValue;         \
+    }
+
 #define QDL_SWITCH_MODE(mode, BODY)                   \
     switch (mode) {                                   \
         case qdl::kDense: { BODY(qdl::kDense); } break;     \

@@ -10,7 +10,7 @@
 namespace qdl {
 hipError_t purified_fwd_launch(int dtype, const PurArgs& a, hipStream_t s);
 hipError_t purified_bwd_launch(int dtype, const PurArgs& a, hipStream_t s);
-int64_t purified_bwd_workspace_bytes(int64_t B, int64_t H, int64_t T, int64_t D);
+int64_t purified_bwd_workspace_bytes(int dtype, int64_t B, int64_t H, int64_t T, int64_t D);
 }  // namespace qdl
 
 namespace {
@@ -71,9 +71,8 @@ int qdl_flash_purified_born_fwd(int dtype, int64_t B, int64_t H, int64_t T, int6
 }
 
 int64_t qdl_flash_purified_born_bwd_workspace_size(int dtype, int64_t B, int64_t H, int64_t T, int64_t D) {
-    (void)dtype;
     if (B <= 0 || H <= 0 || T <= 0 || D <= 0) return 256;
-    return qdl::purified_bwd_workspace_bytes(B, H, T, D);
+    return qdl::purified_bwd_workspace_bytes(dtype, B, H, T, D);
 }
 
 int qdl_flash_purified_born_bwd(int dtype, int64_t B, int64_t H, int64_t T, int64_t D, const void* q,
@@ -95,7 +94,7 @@ int qdl_flash_purified_born_bwd(int dtype, int64_t B, int64_t H, int64_t T, int6
     if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(out) || !aligned16(dout) ||
         !aligned16(dq) || !aligned16(dk) || !aligned16(dv))
         return QDL_BORN_E_ALIGN;
-    const int64_t need = qdl::purified_bwd_workspace_bytes(B, H, T, D);
+    const int64_t need = qdl::purified_bwd_workspace_bytes(dtype, B, H, T, D);
     if (!workspace || workspace_bytes < need) return QDL_BORN_E_WORKSPACE;
     if (!aligned16(workspace)) return QDL_BORN_E_ALIGN;
     qdl::PurArgs a = {};
