@@ -182,6 +182,56 @@ int qdl_flash_purified_born_bwd(int dtype, int64_t B, int64_t H, int64_t T,
                                 qdl_stream_t stream);
 
 /*
+ * Struct form of the forward and backward, for hosts that call often: one
+ * argument block (every field 8 bytes, so it can be packed from a script) in
+ * place of 17 to 26 arguments, and
+ *   - scale == NULL takes scale_value for every head (likewise tau), so a
+ *     plain number needs no device copy and no synchronisation;
+ *   - dscale / dtau == NULL: that gradient is not wanted, and the launches
+ *     that reduce it are left out;
+ *   - purified != 0 selects the purified weights (out is then fp32), prologue
+ *     != 0 the fused Q/K prologue (Born forward).
+ * Other fields, results and return codes are those of the positional entry
+ * points; struct_bytes must be sizeof(qdl_born_call) (else QDL_BORN_E_SHAPE).
+ * Unused fields are ignored.
+ */
+typedef struct qdl_born_call {
+    int64_t struct_bytes;
+    int64_t dtype, B, H, T, D;
+    const void *q, *k, *v;
+    void *out; /* written by the forward, read by the backward */
+    float *z;
+    const float *scale;
+    int64_t n_scale;
+    double scale_value;
+    const int32_t *doc_ids;
+    int64_t is_causal, window_size;
+    double eps;
+    int64_t purified;
+    const float *tau;
+    int64_t n_tau;
+    double tau_value;
+    double eps_base;
+    /* backward */
+    const void *dout;
+    void *dq, *dk, *dv;
+    float *dscale, *dtau;
+    void *workspace; /* the positional entry points' size functions */
+    int64_t workspace_bytes;
+    /* forward of the fused Q/K prologue (qdl_flash_born_fwd_qk_prologue) */
+    int64_t prologue; /* != 0: q, k are raw rows, the fields below apply */
+    int64_t q_strides[3], k_strides[3];
+    const float *cos_table, *sin_table;
+    int64_t n_freq, table_ld;
+    double norm_eps;
+    void *q_out, *k_out;
+    float *q_rinv, *k_rinv;
+} qdl_born_call;
+
+int qdl_flash_born_forward_call(const qdl_born_call *call, qdl_stream_t stream);
+int qdl_flash_born_backward_call(const qdl_born_call *call, qdl_stream_t stream);
+
+/*
  * Q/K prologue of SubspaceProjectorBornAttention.forward (attention.py:573-589,
  * without the optional wave filter and partial key offset), fused into one
  * pass per tensor:

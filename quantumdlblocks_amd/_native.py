@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import struct
 import threading
 from pathlib import Path
 
@@ -33,6 +34,8 @@ EXPORTED_SYMBOLS = (
     "qdl_flash_born_bwd_workspace_size",
     "qdl_flash_born_bwd",
     "qdl_flash_born_bwd_noalloc",
+    "qdl_flash_born_forward_call",
+    "qdl_flash_born_backward_call",
     "qdl_flash_purified_born_fwd",
     "qdl_flash_purified_born_bwd_workspace_size",
     "qdl_flash_purified_born_bwd",
@@ -44,6 +47,23 @@ EXPORTED_SYMBOLS = (
 
 class NativeLibraryError(RuntimeError):
     """The HIP library is missing, failed to load, or returned an error."""
+
+
+# qdl_born_call: every field 8 bytes ("q" integers and addresses, "d" doubles).
+# The forward leaves the backward's fields zero.
+_CALL = struct.Struct("@" + "q" * 6 + "q" * 5 + "qqd" + "qqqd" + "qqqdd" + "q" * 8 + "q" + "q" * 6 + "qqqqd" + "q" * 4)
+_NO_PROLOGUE = (0,) * 7 + (0, 0, 0, 0, 0.0) + (0,) * 4
+
+
+def pack_call(dtype, B, H, T, D, q, k, v, out, z, scale, n_scale, scale_value, doc, causal, window, eps,
+              purified=0, tau=0, n_tau=0, tau_value=0.0, eps_base=0.0,
+              dout=0, dq=0, dk=0, dv=0, dscale=0, dtau=0, workspace=0, workspace_bytes=0,
+              prologue=_NO_PROLOGUE) -> bytes:
+    """The argument block of qdl_flash_born_forward_call / _backward_call;
+    ``prologue``: the fields from ``prologue`` on."""
+    return _CALL.pack(_CALL.size, dtype, B, H, T, D, q, k, v, out, z, scale, n_scale, scale_value, doc, causal, window,
+                      eps, purified, tau, n_tau, tau_value, eps_base, dout, dq, dk, dv, dscale, dtau, workspace,
+                      workspace_bytes, *prologue)
 
 
 _lock = threading.Lock()
@@ -89,6 +109,9 @@ def _bind(lib: ctypes.CDLL) -> None:
         _int, _i64, _dbl,                  # is_causal, window_size, eps
         _ptr, _ptr, _ptr, _ptr, _ptr,      # dq, dk, dv, dscale, stream
     ]
+    for call in (lib.qdl_flash_born_forward_call, lib.qdl_flash_born_backward_call):
+        call.restype = _int
+        call.argtypes = [ctypes.c_char_p, _ptr]  # the packed qdl_born_call, stream
     lib.qdl_flash_purified_born_fwd.restype = _int
     lib.qdl_flash_purified_born_fwd.argtypes = [
         _int, _i64, _i64, _i64, _i64,      # dtype, B, H, T, D

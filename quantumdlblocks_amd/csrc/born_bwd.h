@@ -144,7 +144,7 @@ void born_bwd_dq16_kernel(typename std::conditional<PUR, PurArgs, BwdArgs>::type
     const uint16_t* __restrict__ dO = reinterpret_cast<const uint16_t*>(p.dout) + base;
     const int32_t* __restrict__ docb = has_doc ? p.doc + (size_t)b * T : nullptr;
 
-    const float sc = p.scale[p.per_head_scale ? h : 0];
+    const float sc = arg_scale(p, h);
     const uint32_t flip = (!PUR && sc < 0.f) ? 0x80008000u : 0u;
     // fp16 scales the overlap by c = 2|s|, so the dS operand is the
     // reference's 2 a dP (see E::kScaleInSquare); the epilogue divides c out.
@@ -156,7 +156,7 @@ void born_bwd_dq16_kernel(typename std::conditional<PUR, PurArgs, BwdArgs>::type
     float pg = 0.f, pgt = 0.f, p4g = 0.f, p2e = 0.f;
     if constexpr (PUR) {
         pg = sc;
-        pgt = -sc * p.tau[p.per_head_tau ? h : 0];
+        pgt = -sc * arg_tau(p, h);
         p4g = 4.f * sc;
         p2e = 2.f * p.eps_base;
     }
@@ -449,7 +449,7 @@ void born_bwd_dkdv16_kernel(typename std::conditional<PUR, PurArgs, BwdArgs>::ty
     const float* __restrict__ NDl = p.ndelta + (size_t)bh * T;
     const int32_t* __restrict__ docb = has_doc ? p.doc + (size_t)b * T : nullptr;
 
-    const float sc = p.scale[p.per_head_scale ? h : 0];
+    const float sc = arg_scale(p, h);
     const uint32_t flip = (!PUR && sc < 0.f) ? 0x80008000u : 0u;
     // fp16 scales the overlap by c = 2|s|, so the dS operand is the
     // reference's 2 a dP (see E::kScaleInSquare); the epilogue divides c out.
@@ -460,7 +460,7 @@ void born_bwd_dkdv16_kernel(typename std::conditional<PUR, PurArgs, BwdArgs>::ty
     };
     float pg = 0.f, pgt = 0.f, ptau = 0.f, p4g = 0.f, p2e = 0.f, pe = 0.f;
     if constexpr (PUR) {
-        ptau = p.tau[p.per_head_tau ? h : 0];
+        ptau = arg_tau(p, h);
         pg = sc;
         pgt = -sc * ptau;
         p4g = 4.f * sc;
@@ -757,7 +757,7 @@ void born_bwd_dq32_kernel(BwdArgs p) {
     const float* __restrict__ dO = reinterpret_cast<const float*>(p.dout) + base;
     const int32_t* __restrict__ docb = has_doc ? p.doc + (size_t)b * T : nullptr;
 
-    const float sc = p.scale[p.per_head_scale ? h : 0];
+    const float sc = arg_scale(p, h);
     const float sgn = (sc < 0.f) ? -1.f : 1.f;
 
     f32x4 qr[KQ], dr[KQ];
@@ -955,7 +955,7 @@ void born_bwd_dkdv32_kernel(BwdArgs p) {
     const float* __restrict__ NDl = p.ndelta + (size_t)bh * T;
     const int32_t* __restrict__ docb = has_doc ? p.doc + (size_t)b * T : nullptr;
 
-    const float sc = p.scale[p.per_head_scale ? h : 0];
+    const float sc = arg_scale(p, h);
     const float sgn = (sc < 0.f) ? -1.f : 1.f;
 
     // B operands: K'[key][d(t, g)], V[key][d(t, g)] with d(t, g) = 8(t/4) + 4g + t%4.
@@ -1210,9 +1210,7 @@ hipError_t launch_bwd16(const BwdArgs& a, hipStream_t st) {
                 if ((e = launch_bwd16_dkdv_fast<E, 64, kWindowNC>(a, st)) != hipSuccess) return e;
             }
             const int nwg = ((a.T + 255) / 256) * a.B * a.H;
-            hipLaunchKernelGGL(born_bwd_dscale_groups_kernel<0>, dim3((unsigned)(a.per_head_scale ? a.H : 1)), dim3(256),
-                               0, st, a, nwg);
-            return hipGetLastError();
+            return launch_dscale_groups(a, nwg, st);
         }
     }
     // Documents (with or without a causal window): the same two fast
@@ -1232,9 +1230,7 @@ hipError_t launch_bwd16(const BwdArgs& a, hipStream_t st) {
             }
             if (e != hipSuccess) return e;
             const int nwg = bwd16_dq_fast_groups(a.B, a.H, a.T, true);
-            hipLaunchKernelGGL(born_bwd_dscale_groups_kernel<0>, dim3((unsigned)(a.per_head_scale ? a.H : 1)), dim3(256),
-                               0, st, a, nwg);
-            return hipGetLastError();
+            return launch_dscale_groups(a, nwg, st);
         }
     }
     // D == 128, dense, causal or a sliding window with or without causality
@@ -1285,9 +1281,7 @@ hipError_t launch_bwd16(const BwdArgs& a, hipStream_t st) {
             if ((e = launch_bwd16_dq_fast<E, 64, MODE>(a, st)) != hipSuccess) return e;
             if ((e = launch_bwd16_dkdv_fast<E, 64, MODE>(a, st)) != hipSuccess) return e;
             const int nwg = ((a.T + 255) / 256) * a.B * a.H;
-            hipLaunchKernelGGL(born_bwd_dscale_groups_kernel<0>, dim3((unsigned)(a.per_head_scale ? a.H : 1)), dim3(256),
-                               0, st, a, nwg);
-            return hipGetLastError();
+            return launch_dscale_groups(a, nwg, st);
         }
     }
     if (!fast && (e = launch_bwd_common_pre<E, false>(a, st)) != hipSuccess) return e;

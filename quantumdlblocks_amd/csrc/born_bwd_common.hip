@@ -41,7 +41,7 @@ __global__ __launch_bounds__(64) void born_bwd_dscale_final_kernel(BwdArgs p, co
     if (threadIdx.x != 0) return;
     double acc = 0.0;
     for (int c = 0; c < DSCALE_CHUNKS; ++c) acc += part[out * DSCALE_CHUNKS + c];
-    const float s = p.scale[out];
+    const float s = arg_scale(p, out);
     p.dscale[out] = (s == 0.f) ? 0.f : (float)(2.0 / (double)s * (double)p.eps * acc);
 }
 
@@ -52,6 +52,7 @@ __global__ void born_zero_fill_kernel(float* __restrict__ x, int64_t n) {
 }
 
 hipError_t launch_bwd_common_post(const BwdArgs& a, hipStream_t st) {
+    if (a.dscale == nullptr) return hipSuccess;
     const int nout = a.per_head_scale ? a.H : 1;
     hipLaunchKernelGGL(born_bwd_dscale_partial_kernel, dim3(DSCALE_CHUNKS, nout), dim3(256), 0, st, a,
                        a.dscale_part);

@@ -102,14 +102,14 @@ void born_bwd16_dq_d128_kernel(typename std::conditional<PUR, PurArgs, BwdArgs>:
     const int D = PAD ? p.D : DP;
     const int CG = D / 8;
     const size_t base = (size_t)bh * T * D;
-    const float sc = p.scale[p.per_head_scale ? h : 0];
+    const float sc = arg_scale(p, h);
     const uint32_t flip = (!PUR && sc < 0.f) ? 0x80008000u : 0u;
     const float sq_pre = (E::kScaleInSquare && sc != 0.f) ? 2.f * fabsf(sc) : 1.f;
     // Purified: t = gamma r - gamma tau; dR / dP = 4 gamma u^3 + 2 eps_base b.
     float pg = 0.f, pgt = 0.f, p4g = 0.f, p2e = 0.f;
     if constexpr (PUR) {
         pg = sc;
-        pgt = -sc * p.tau[p.per_head_tau ? h : 0];
+        pgt = -sc * arg_tau(p, h);
         p4g = 4.f * sc;
         p2e = 2.f * p.eps_base;
     }
@@ -567,12 +567,12 @@ void born_bwd16_dkdv_d128_kernel(typename std::conditional<PUR, PurArgs, BwdArgs
     const int D = PAD ? p.D : DP;
     const int CG = D / 8;
     const size_t base = (size_t)bh * T * D;
-    const float sc = p.scale[p.per_head_scale ? h : 0];
+    const float sc = arg_scale(p, h);
     const uint32_t flip = (!PUR && sc < 0.f) ? 0x80008000u : 0u;
     const float sq_pre = (E::kScaleInSquare && sc != 0.f) ? 2.f * fabsf(sc) : 1.f;
     float pg = 0.f, pgt = 0.f, ptau = 0.f, p4g = 0.f, p2e = 0.f, pe = 0.f;
     if constexpr (PUR) {
-        ptau = p.tau[p.per_head_tau ? h : 0];
+        ptau = arg_tau(p, h);
         pg = sc;
         pgt = -sc * ptau;
         p4g = 4.f * sc;
@@ -1088,9 +1088,7 @@ hipError_t launch_bwd16_d128(const BwdArgs& a, hipStream_t st) {
     hipLaunchKernelGGL((born_bwd16_dkdv_d128_kernel<E, MODE, false, PAD, DOC, NWK>), dim3(nk * BH), dim3(NWK * 64), 0,
                        st, a);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    hipLaunchKernelGGL(born_bwd_dscale_groups_kernel<0>, dim3((unsigned)(a.per_head_scale ? a.H : 1)), dim3(256), 0,
-                       st, a, (int)(nq * BH));
-    return hipGetLastError();
+    return launch_dscale_groups(a, (int)(nq * BH), st);
 }
 
 // The purified D == 128 backward (bf16 or fp16): dQ (and the workspace),

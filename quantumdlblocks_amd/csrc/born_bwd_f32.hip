@@ -24,10 +24,7 @@ hipError_t bwd_launch_f32(const BwdArgs& a, hipStream_t s) {
 hipError_t purified_bwd_f32_launch(const PurArgs& a, hipStream_t s) {
     const hipError_t e = launch_f32_bwd<true>(a, s);
     if (e != hipSuccess) return e;
-    const int n_scale = a.per_head_scale ? a.H : 1, n_tau = a.per_head_tau ? a.H : 1;
-    hipLaunchKernelGGL(purified_param_reduce_kernel<0>, dim3((unsigned)(n_scale + n_tau)), dim3(256), 0, s, a,
-                       f32_groups(a.B, a.H, a.T), n_scale);
-    return hipGetLastError();
+    return launch_purified_param_reduce(a, f32_groups(a.B, a.H, a.T), s);
 }
 
 }  // namespace qdl

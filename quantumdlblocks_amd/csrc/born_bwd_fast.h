@@ -193,7 +193,7 @@ void born_bwd16_dq_fast_kernel(typename std::conditional<PUR, PurArgs, BwdArgs>:
     const int D = PAD ? p.D : DP;
     const int CG = D / 8;
     const size_t base = (size_t)bh * T * D;
-    const float sc = p.scale[p.per_head_scale ? h : 0];
+    const float sc = arg_scale(p, h);
     const uint32_t flip = (!PUR && sc < 0.f) ? 0x80008000u : 0u;
     // fp16 scales the overlap by c = 2|s|, so the dS operand is the
     // reference's 2 a dP (see E::kScaleInSquare); the epilogue divides c out.
@@ -202,7 +202,7 @@ void born_bwd16_dq_fast_kernel(typename std::conditional<PUR, PurArgs, BwdArgs>:
     float pg = 0.f, pgt = 0.f, p4g = 0.f, p2e = 0.f;
     if constexpr (PUR) {
         pg = sc;
-        pgt = -sc * p.tau[p.per_head_tau ? h : 0];
+        pgt = -sc * arg_tau(p, h);
         p4g = 4.f * sc;
         p2e = 2.f * p.eps_base;
     }
@@ -718,9 +718,16 @@ __global__ __launch_bounds__(256) void born_bwd_dscale_groups_kernel(BwdArgs p, 
         __syncthreads();
     }
     if (threadIdx.x == 0) {
-        const float s = p.scale[o];
+        const float s = arg_scale(p, o);
         p.dscale[o] = (s == 0.f) ? 0.f : (float)(2.0 / (double)s * (double)p.eps * red[0]);
     }
+}
+
+inline hipError_t launch_dscale_groups(const BwdArgs& a, int nwg, hipStream_t st) {
+    if (a.dscale == nullptr) return hipSuccess;  // the scale needs no gradient
+    hipLaunchKernelGGL(born_bwd_dscale_groups_kernel<0>, dim3((unsigned)(a.per_head_scale ? a.H : 1)), dim3(256), 0, st,
+                       a, nwg);
+    return hipGetLastError();
 }
 
 // Workgroups of the D = 64 dQ launch (each writes one dscale partial):
@@ -816,12 +823,12 @@ void born_bwd16_dkdv_fast_kernel(typename std::conditional<PUR, PurArgs, BwdArgs
     const int D = PAD ? p.D : DP;
     const int CG = D / 8;
     const size_t base = (size_t)bh * T * D;
-    const float sc = p.scale[p.per_head_scale ? h : 0];
+    const float sc = arg_scale(p, h);
     const uint32_t flip = (!PUR && sc < 0.f) ? 0x80008000u : 0u;
     const float sq_pre = (E::kScaleInSquare && sc != 0.f) ? 2.f * fabsf(sc) : 1.f;
     float pg = 0.f, pgt = 0.f, ptau = 0.f, p4g = 0.f, p2e = 0.f, pe = 0.f;
     if constexpr (PUR) {
-        ptau = p.tau[p.per_head_tau ? h : 0];
+        ptau = arg_tau(p, h);
         pg = sc;
         pgt = -sc * ptau;
         p4g = 4.f * sc;

@@ -31,6 +31,59 @@ int hip_status(hipError_t e) { return e == hipSuccess ? QDL_BORN_OK : (int)e; }
 
 }  // namespace
 
+namespace qdl {
+
+int fwd_with_prologue(int dtype, const FwdArgs& a, const ProloguePlan& p, hipStream_t s) {
+    const int64_t T = a.T, D = a.D;
+    // bf16, D = 64, dense or causal, with or without document ids (with
+    // documents also a causal window): K is normalised by the prologue kernel
+    // (K alone), then one attention kernel normalises each query block as it
+    // loads it (raw rows 16-byte aligned, (T + 256) rows of their time stride
+    // within 32-bit offsets) and, when q_rinv is given (a backward follows),
+    // writes the normalised rows and their 1/norm.
+    const bool q_rows_ok = aligned16(a.q) && p.q_strides[0] % 8 == 0 && p.q_strides[1] % 8 == 0 &&
+                           p.q_strides[2] % 8 == 0 && p.q_strides[2] >= D &&
+                           (T + 256) * p.q_strides[2] * 2 < ((int64_t)1 << 31);
+    const bool masks_ok = a.doc ? (a.window == 0 || a.is_causal) : a.window == 0;
+    if (dtype == QDL_BORN_DTYPE_BF16 && D == 64 && masks_ok && q_rows_ok && (!p.cos || p.n_freq >= 1) &&
+        (T + 256) * D * 2 < ((int64_t)1 << 31)) {
+        const int rc = qdl_flash_born_qk_prologue_fwd(dtype, a.B, a.H, T, D, nullptr, nullptr, a.k, p.k_strides, p.cos,
+                                                      p.sin, p.n_freq, p.table_ld, p.norm_eps, nullptr, p.k_out,
+                                                      nullptr, p.k_rinv, reinterpret_cast<qdl_stream_t>(s));
+        if (rc != QDL_BORN_OK) return rc;
+        FwdProArgs f = {};
+        static_cast<FwdArgs&>(f) = a;
+        f.k = p.k_out;
+        f.q_sb = p.q_strides[0];
+        f.q_sh = p.q_strides[1];
+        f.q_st = p.q_strides[2];
+        f.cos = p.cos;
+        f.sin = p.cos ? p.sin : nullptr;
+        f.ld = (int)p.table_ld;
+        f.nfreq = (int)p.n_freq;
+        f.norm_eps = (float)p.norm_eps;
+        f.q_out = p.q_out;
+        f.q_rinv = p.q_rinv;
+        return hip_status(fwd_prologue_launch_bf16(f, s));
+    }
+    // Every other case: the prologue kernel, then the attention kernels on
+    // its output (the same rows and results, two launches).
+    const int rc = qdl_flash_born_qk_prologue_fwd(dtype, a.B, a.H, T, D, a.q, p.q_strides, a.k, p.k_strides, p.cos,
+                                                  p.sin, p.n_freq, p.table_ld, p.norm_eps, p.q_out, p.k_out, p.q_rinv,
+                                                  p.k_rinv, reinterpret_cast<qdl_stream_t>(s));
+    if (rc != QDL_BORN_OK) return rc;
+    FwdArgs f = a;
+    f.q = p.q_out;
+    f.k = p.k_out;
+    switch (dtype) {
+        case QDL_BORN_DTYPE_BF16: return hip_status(fwd_launch_bf16(f, s));
+        case QDL_BORN_DTYPE_F16: return hip_status(fwd_launch_f16(f, s));
+        default: return hip_status(fwd_launch_f32(f, s));
+    }
+}
+
+}  // namespace qdl
+
 extern "C" {
 
 const char* qdl_flash_born_version(void) { return "qdl_flash_born 0.1.0 gfx950"; }
@@ -169,57 +222,25 @@ int qdl_flash_born_fwd_qk_prologue(int dtype, int64_t B, int64_t H, int64_t T, i
     if (!q || !k || !v || !q_strides || !k_strides || !out || !z || !scale || !q_out || !k_out)
         return QDL_BORN_E_NULL;
     if (!aligned16(v) || !aligned16(out) || !aligned16(q_out) || !aligned16(k_out)) return QDL_BORN_E_ALIGN;
-    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    // bf16, D = 64, dense or causal, with or without document ids (with
-    // documents also a causal window): K is normalised by the prologue kernel
-    // (K alone), then one attention kernel normalises each query block as it
-    // loads it (raw rows 16-byte aligned, (T + 256) rows of their time stride
-    // within 32-bit offsets) and, when q_rinv is given (a backward follows),
-    // writes the normalised rows and their 1/norm.
-    const bool q_rows_ok = aligned16(q) && q_strides[0] % 8 == 0 && q_strides[1] % 8 == 0 &&
-                           q_strides[2] % 8 == 0 && q_strides[2] >= D &&
-                           (T + 256) * q_strides[2] * 2 < ((int64_t)1 << 31);
-    const bool masks_ok = doc_ids ? (window_size == 0 || is_causal) : window_size == 0;
-    if (dtype == QDL_BORN_DTYPE_BF16 && D == 64 && masks_ok && q_rows_ok &&
-        (!cos_table || n_freq >= 1) && (T + 256) * D * 2 < ((int64_t)1 << 31)) {
-        rc = qdl_flash_born_qk_prologue_fwd(dtype, B, H, T, D, nullptr, nullptr, k, k_strides, cos_table, sin_table,
-                                            n_freq, table_ld, norm_eps, nullptr, k_out, nullptr, k_rinv, stream);
-        if (rc != QDL_BORN_OK) return rc;
-        qdl::FwdProArgs a;
-        a.q = q;
-        a.k = k_out;
-        a.v = v;
-        a.o = out;
-        a.z = z;
-        a.scale = scale;
-        a.doc = doc_ids;
-        a.per_head_scale = n_scale > 1 ? 1 : 0;
-        a.B = (int)B;
-        a.H = (int)H;
-        a.T = (int)T;
-        a.D = (int)D;
-        a.is_causal = is_causal ? 1 : 0;
-        a.window = (int)window_size;
-        a.eps = (float)eps;
-        a.q_sb = q_strides[0];
-        a.q_sh = q_strides[1];
-        a.q_st = q_strides[2];
-        a.cos = cos_table;
-        a.sin = cos_table ? sin_table : nullptr;
-        a.ld = (int)table_ld;
-        a.nfreq = (int)n_freq;
-        a.norm_eps = (float)norm_eps;
-        a.q_out = q_out;
-        a.q_rinv = q_rinv;
-        return hip_status(qdl::fwd_prologue_launch_bf16(a, s));
-    }
-    // Every other case: the prologue kernel, then the attention kernels on
-    // its output (the same rows and results, two launches).
-    rc = qdl_flash_born_qk_prologue_fwd(dtype, B, H, T, D, q, q_strides, k, k_strides, cos_table, sin_table,
-                                        n_freq, table_ld, norm_eps, q_out, k_out, q_rinv, k_rinv, stream);
-    if (rc != QDL_BORN_OK) return rc;
-    return qdl_flash_born_fwd(dtype, B, H, T, D, q_out, k_out, v, out, z, scale, n_scale, doc_ids, is_causal,
-                              window_size, eps, stream);
+    qdl::FwdArgs a = {};
+    a.q = q;
+    a.k = k;
+    a.v = v;
+    a.o = out;
+    a.z = z;
+    a.scale = scale;
+    a.doc = doc_ids;
+    a.per_head_scale = n_scale > 1 ? 1 : 0;
+    a.B = (int)B;
+    a.H = (int)H;
+    a.T = (int)T;
+    a.D = (int)D;
+    a.is_causal = is_causal ? 1 : 0;
+    a.window = (int)window_size;
+    a.eps = (float)eps;
+    const qdl::ProloguePlan p = {q_strides, k_strides, cos_table, sin_table, n_freq, table_ld,
+                                 norm_eps,  q_out,     k_out,     q_rinv,    k_rinv};
+    return qdl::fwd_with_prologue(dtype, a, p, reinterpret_cast<hipStream_t>(stream));
 }
 
 }  // extern "C"

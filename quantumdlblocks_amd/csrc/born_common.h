@@ -215,6 +215,17 @@ __device__ __forceinline__ f32x16 zero16() {
     return z;
 }
 
+// A head's scale and tau: from device memory, or, without a pointer, the value
+// in the argument block (a caller's plain float needs no device copy).
+template <class Args>
+__device__ __forceinline__ float arg_scale(const Args& p, int h) {
+    return p.scale != nullptr ? p.scale[p.per_head_scale ? h : 0] : p.scale_value;
+}
+template <class Args>
+__device__ __forceinline__ float arg_tau(const Args& p, int h) {
+    return p.tau != nullptr ? p.tau[p.per_head_tau ? h : 0] : p.tau_value;
+}
+
 // Kernel argument block shared by the forward kernels.
 struct FwdArgs {
     const void* q;
@@ -222,7 +233,8 @@ struct FwdArgs {
     const void* v;
     void* o;
     float* z;
-    const float* scale;
+    const float* scale;  // 1 or H values, or nullptr: scale_value
+    float scale_value;
     const int32_t* doc;  // (B, T) or nullptr
     int per_head_scale;
     int B, H, T, D;
@@ -254,7 +266,8 @@ struct BwdArgs {
     const void* o;
     const void* dout;
     const float* z;
-    const float* scale;
+    const float* scale;  // 1 or H values, or nullptr: scale_value
+    float scale_value;
     const int32_t* doc;
     void* dq;
     void* dk;
@@ -263,7 +276,7 @@ struct BwdArgs {
     float* delta_z;        // (B, H, T) workspace: dO . O / Z per row
     float* zinv;           // (B, H, T) workspace: 1 / Z per row
     double* dscale_part;   // workspace: dscale partial sums (per chunk of rows, or per workgroup)
-    float* dscale;         // n_scale outputs
+    float* dscale;         // n_scale outputs, or nullptr: not wanted
     int per_head_scale;
     int B, H, T, D;
     int is_causal;

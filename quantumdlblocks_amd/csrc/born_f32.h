@@ -183,8 +183,8 @@ struct F32Weights {
     float gam = 0.f, tau = 0.f, eb = 0.f;
     __device__ __forceinline__ F32Weights(const Args& p, int h) {
         if constexpr (PUR) {
-            gam = p.scale[p.per_head_scale ? h : 0];
-            tau = p.tau[p.per_head_tau ? h : 0];
+            gam = arg_scale(p, h);
+            tau = arg_tau(p, h);
             eb = p.eps_base;
         }
     }
@@ -221,7 +221,7 @@ void born_f32_fwd_kernel(typename std::conditional<PUR, PurArgs, FwdArgs>::type 
     const float* __restrict__ K = reinterpret_cast<const float*>(p.k) + base;
     const float* __restrict__ V = reinterpret_cast<const float*>(p.v) + base;
     const int32_t* __restrict__ docb = m.has_doc ? p.doc + (size_t)b * T : nullptr;
-    const float sc = p.scale[p.per_head_scale ? h : 0];
+    const float sc = arg_scale(p, h);
     const F32Weights<PUR, Args> pw(p, h);
 
     int t_lo = 0, t_hi = ((m.causal ? min(T, m0 + kF32Rows) : T) + 31) / 32 - 1;  // first and last key tile
@@ -389,7 +389,7 @@ void born_f32_dq_kernel(typename std::conditional<PUR, PurArgs, BwdArgs>::type p
         Zr = p.z + (size_t)blk.bh * T;
     }
     const int32_t* __restrict__ docb = m.has_doc ? p.doc + (size_t)b * T : nullptr;
-    const float sc = p.scale[p.per_head_scale ? h : 0];
+    const float sc = arg_scale(p, h);
     const F32Weights<PUR, Args> pw(p, h);
 
     int t_lo = 0, t_hi = ((m.causal ? min(T, m0 + kF32Rows) : T) + 31) / 32 - 1;
@@ -551,7 +551,7 @@ void born_f32_dkdv_kernel(typename std::conditional<PUR, PurArgs, BwdArgs>::type
     const float* __restrict__ NDl = p.ndelta + (size_t)blk.bh * T;
     const float* __restrict__ ZIl = p.zinv + (size_t)blk.bh * T;
     const int32_t* __restrict__ docb = m.has_doc ? p.doc + (size_t)b * T : nullptr;
-    const float sc = p.scale[p.per_head_scale ? h : 0];
+    const float sc = arg_scale(p, h);
     const F32Weights<PUR, Args> pw(p, h);
 
     int t_lo = m.causal ? blk.mb : 0, t_hi = (T + 31) / 32 - 1;  // first and last query tile

@@ -103,7 +103,7 @@ void born_fwd16_kernel(typename std::conditional<PUR, PurArgs, FwdArgs>::type p)
     const uint16_t* __restrict__ V = reinterpret_cast<const uint16_t*>(p.v) + base;
     const int32_t* __restrict__ docb = has_doc ? p.doc + (size_t)b * T : nullptr;
 
-    const float sc = p.scale[p.per_head_scale ? h : 0];
+    const float sc = arg_scale(p, h);
     const uint32_t flip = (!PUR && sc < 0.f) ? 0x80008000u : 0u;  // sign of the scale folded into Q
     // fp16: the weights are the reference's relu(s r)^2 (c = |s| times the
     // sign-folded overlap; born_weight_pair); bf16: s^2 goes back in per row.
@@ -112,7 +112,7 @@ void born_fwd16_kernel(typename std::conditional<PUR, PurArgs, FwdArgs>::type p)
     float pg = 0.f, pgt = 0.f, pse = 0.f;
     if constexpr (PUR) {
         pg = sc;
-        pgt = -sc * p.tau[p.per_head_tau ? h : 0];
+        pgt = -sc * arg_tau(p, h);
         pse = sqrtf(p.eps_base);
     }
 
@@ -532,7 +532,7 @@ void born_fwd32_kernel(FwdArgs p) {
     const float* __restrict__ V = reinterpret_cast<const float*>(p.v) + base;
     const int32_t* __restrict__ docb = has_doc ? p.doc + (size_t)b * T : nullptr;
 
-    const float sc = p.scale[p.per_head_scale ? h : 0];
+    const float sc = arg_scale(p, h);
     const float sgn = (sc < 0.f) ? -1.f : 1.f;
 
     // Contraction step t of the QK product uses dim 8*(t/4) + 4*g + (t%4), so

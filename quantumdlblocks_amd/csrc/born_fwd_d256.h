@@ -85,7 +85,7 @@ void born_fwd16_d256_kernel(typename std::conditional<PUR, PurArgs, FwdArgs>::ty
     const int D = PAD ? p.D : DP;
     const int CG = D / 8;
     const size_t base = (size_t)bh * T * D;
-    const float sc = p.scale[p.per_head_scale ? h : 0];
+    const float sc = arg_scale(p, h);
     const uint32_t flip = (!PUR && sc < 0.f) ? 0x80008000u : 0u;  // sign of the scale folded into Q
     // fp16: the reference's weights relu(s r)^2 (born_weight_pair).
     const float sq_pre = E::kScaleInSquare ? fabsf(sc) : 1.f;
@@ -93,7 +93,7 @@ void born_fwd16_d256_kernel(typename std::conditional<PUR, PurArgs, FwdArgs>::ty
     float pg = 0.f, pgt = 0.f, pse = 0.f;
     if constexpr (PUR) {
         pg = sc;
-        pgt = -sc * p.tau[p.per_head_tau ? h : 0];
+        pgt = -sc * arg_tau(p, h);
         pse = sqrtf(p.eps_base);
     }
 

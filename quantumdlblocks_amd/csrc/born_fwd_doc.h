@@ -110,7 +110,7 @@ void born_fwd16_doc_kernel(
     const size_t base = (size_t)bh * T * DP;
     const uint16_t* __restrict__ Qg = reinterpret_cast<const uint16_t*>(p.q) + base;
     const int32_t* __restrict__ docb = p.doc + (size_t)b * T;
-    const float sc = p.scale[p.per_head_scale ? h : 0];
+    const float sc = arg_scale(p, h);
     const uint32_t flip = (!PUR && sc < 0.f) ? 0x80008000u : 0u;  // sign of the scale folded into Q
     // fp16: the reference's weights relu(s r)^2 (born_weight_pair).
     const float sq_pre = E::kScaleInSquare ? fabsf(sc) : 1.f;
@@ -118,7 +118,7 @@ void born_fwd16_doc_kernel(
     float pg = 0.f, pgt = 0.f, pse = 0.f;
     if constexpr (PUR) {
         pg = sc;
-        pgt = -sc * p.tau[p.per_head_tau ? h : 0];
+        pgt = -sc * arg_tau(p, h);
         pse = sqrtf(p.eps_base);
     }
 

@@ -214,13 +214,13 @@ void born_fwd16_fast_kernel(
     const int RBG = 2 * D;
     const int CG = D / 8;
     const size_t base = (size_t)bh * T * D;
-    const float sc = p.scale[p.per_head_scale ? h : 0];
+    const float sc = arg_scale(p, h);
     const uint32_t flip = (!PUR && sc < 0.f) ? 0x80008000u : 0u;  // sign of the scale folded into Q
     // Purified weights: t = gamma r - gamma tau, b' = sqrt(eps_base) relu(r).
     float pg = 0.f, pgt = 0.f, pse = 0.f;
     if constexpr (PUR) {
         pg = sc;
-        pgt = -sc * p.tau[p.per_head_tau ? h : 0];
+        pgt = -sc * arg_tau(p, h);
         pse = sqrtf(p.eps_base);
     }
     // fp16: the weights are the reference's relu(s r)^2 (c = |s| times the

@@ -22,6 +22,18 @@ hipError_t bwd_launch_bf16(const BwdArgs& a, hipStream_t s);
 // The forward with the Q/K prologue fused into its loads (bf16, D == 64, dense
 // or causal); hipErrorInvalidValue for anything else.
 hipError_t fwd_prologue_launch_bf16(const FwdProArgs& a, hipStream_t s);
+// The Q/K prologue and then the forward, on checked arguments (born_capi.hip):
+// `a` holds the attention's (q, k the raw rows), `p` the prologue's.  Returns a
+// QDL_BORN code or a hipError_t.
+struct ProloguePlan {
+    const int64_t *q_strides, *k_strides;
+    const float *cos, *sin;
+    int64_t n_freq, table_ld;
+    double norm_eps;
+    void *q_out, *k_out;
+    float *q_rinv, *k_rinv;
+};
+int fwd_with_prologue(int dtype, const FwdArgs& a, const ProloguePlan& p, hipStream_t s);
 hipError_t bwd_launch_f16(const BwdArgs& a, hipStream_t s);
 hipError_t bwd_launch_f32(const BwdArgs& a, hipStream_t s);
 

@@ -159,8 +159,8 @@ void purified_fwd_kernel(PurArgs p) {
 
     const size_t base = (size_t)bh * T * D;
     const int32_t* __restrict__ docb = has_doc ? p.doc + (size_t)b * T : nullptr;
-    const float gam = p.scale[p.per_head_scale ? h : 0];
-    const float tau = p.tau[p.per_head_tau ? h : 0];
+    const float gam = arg_scale(p, h);
+    const float tau = arg_tau(p, h);
     const float eb = p.eps_base;
 
     // Contraction step t of the QK product uses dim 8 (t/4) + 4 g + t%4.
@@ -378,8 +378,8 @@ void purified_dkdv_kernel(PurArgs p) {
     const float* __restrict__ NDl = p.ndelta + (size_t)bh * T;
     const float* __restrict__ ZIl = p.zinv + (size_t)bh * T;
     const int32_t* __restrict__ docb = has_doc ? p.doc + (size_t)b * T : nullptr;
-    const float gam = p.scale[p.per_head_scale ? h : 0];
-    const float tau = p.tau[p.per_head_tau ? h : 0];
+    const float gam = arg_scale(p, h);
+    const float tau = arg_tau(p, h);
     const float eb = p.eps_base;
 
     // B operands: K[key][d(t, g)], V[key][d(t, g)] with d(t, g) = 8 (t/4) + 4 g + t%4.
@@ -621,8 +621,8 @@ void purified_dq_kernel(PurArgs p) {
 
     const size_t base = (size_t)bh * T * D;
     const int32_t* __restrict__ docb = has_doc ? p.doc + (size_t)b * T : nullptr;
-    const float gam = p.scale[p.per_head_scale ? h : 0];
-    const float tau = p.tau[p.per_head_tau ? h : 0];
+    const float gam = arg_scale(p, h);
+    const float tau = arg_tau(p, h);
     const float eb = p.eps_base;
 
     f32x4 qr[KQ], dr[KQ];
@@ -762,7 +762,16 @@ __global__ __launch_bounds__(256) void purified_param_reduce_kernel(PurArgs p, i
         if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
         __syncthreads();
     }
-    if (threadIdx.x == 0) (is_tau ? p.dtau : p.dscale)[o] = (float)red[0];
+    float* const dst = is_tau ? p.dtau : p.dscale;
+    if (threadIdx.x == 0 && dst != nullptr) dst[o] = (float)red[0];
+}
+
+inline hipError_t launch_purified_param_reduce(const PurArgs& a, int nwg, hipStream_t st) {
+    if (a.dscale == nullptr && a.dtau == nullptr) return hipSuccess;  // neither needs a gradient
+    const int n_scale = a.per_head_scale ? a.H : 1, n_tau = a.per_head_tau ? a.H : 1;
+    hipLaunchKernelGGL(purified_param_reduce_kernel<0>, dim3((unsigned)(n_scale + n_tau)), dim3(256), 0, st, a, nwg,
+                       n_scale);
+    return hipGetLastError();
 }
 
 // Workgroups of the dK/dV kernel (the partial-sum count).
@@ -809,9 +818,7 @@ hipError_t launch_purified_bwd(const PurArgs& a, hipStream_t st) {
     hipLaunchKernelGGL((purified_dq_kernel<IN, DP, C::NW, C::BN, C::DQ_WPE>), dim3((unsigned)((a.T + BM - 1) / BM) * BH),
                        dim3(C::NW * 64), 0, st, a);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    const int n_scale = a.per_head_scale ? a.H : 1, n_tau = a.per_head_tau ? a.H : 1;
-    hipLaunchKernelGGL(purified_param_reduce_kernel<0>, dim3((unsigned)(n_scale + n_tau)), dim3(256), 0, st, a, nwg, n_scale);
-    return hipGetLastError();
+    return launch_purified_param_reduce(a, nwg, st);
 }
 
 }  // namespace qdl

@@ -14,13 +14,14 @@ struct PurArgs {
     const float* o_in;   // backward: the forward's fp32 output
     const void* dout;    // backward: upstream gradient, input dtype
     const float* z_in;   // backward: the forward's Z
-    const float* scale;  // gamma: 1 or H values
-    const float* tau;    // tau: 1 or H values
+    const float* scale;  // gamma: 1 or H values, or nullptr: scale_value
+    const float* tau;    // tau: 1 or H values, or nullptr: tau_value
+    float scale_value, tau_value;
     const int32_t* doc;  // (B, T) or nullptr
     void* dq;
     void* dk;
     void* dv;
-    float* dscale;       // n_scale outputs
+    float* dscale;       // n_scale outputs; dscale and dtau nullptr: not wanted
     float* dtau;         // n_tau outputs
     float* ndelta;       // workspace (B, H, T): -delta
     float* zinv;         // workspace (B, H, T): 1 / Z

@@ -23,9 +23,7 @@ static hipError_t purified_bwd_fast(const PurArgs& a, hipStream_t s) {
     hipLaunchKernelGGL((born_bwd16_dkdv_fast_kernel<E, 64, MODE, true, DOC, PAD>), dim3((unsigned)nwg), dim3(256), 0,
                        s, a);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    const int n_scale = a.per_head_scale ? a.H : 1, n_tau = a.per_head_tau ? a.H : 1;
-    hipLaunchKernelGGL(purified_param_reduce_kernel<0>, dim3((unsigned)(n_scale + n_tau)), dim3(256), 0, s, a, nwg, n_scale);
-    return hipGetLastError();
+    return launch_purified_param_reduce(a, nwg, s);
 }
 
 // 16-bit, 64 < D <= 128: the D = 128 dQ and dK/dV kernels' purified mode,
@@ -37,9 +35,7 @@ static hipError_t purified_bwd_d128(const PurArgs& a, hipStream_t s) {
     if (e != hipSuccess) return e;
     // dK/dV workgroups: 128-key blocks, 64-key blocks with documents.
     const int nwg = DOC ? ((a.T + 63) / 64) * a.B * a.H : purified_dkdv_groups(a.B, a.H, a.T, 128);
-    const int n_scale = a.per_head_scale ? a.H : 1, n_tau = a.per_head_tau ? a.H : 1;
-    hipLaunchKernelGGL(purified_param_reduce_kernel<0>, dim3((unsigned)(n_scale + n_tau)), dim3(256), 0, s, a, nwg, n_scale);
-    return hipGetLastError();
+    return launch_purified_param_reduce(a, nwg, s);
 }
 
 template <class IN>
@@ -82,10 +78,7 @@ static hipError_t purified_bwd_dispatch(const PurArgs& a, hipStream_t s) {
         hipError_t e = purified_bwd_d256_launch(E::kDtype, a, s);
         if (e != hipSuccess) return e;
         const int nwg = ((a.T + 127) / 128) * a.B * a.H;
-        const int n_scale = a.per_head_scale ? a.H : 1, n_tau = a.per_head_tau ? a.H : 1;
-        hipLaunchKernelGGL(purified_param_reduce_kernel<0>, dim3((unsigned)(n_scale + n_tau)), dim3(256), 0, s, a, nwg,
-                           n_scale);
-        return hipGetLastError();
+        return launch_purified_param_reduce(a, nwg, s);
     }
     if (k16 && (a.D > 128 || a.doc != nullptr)) return purified_wide_bwd_launch(E::kDtype, a, s);
     if constexpr (!k16) {

@@ -57,10 +57,7 @@ hipError_t wide_bwd(const PurArgs& a, hipStream_t st) {
     hipLaunchKernelGGL((born_bwd_dq16_kernel<E, DP, C::DQ_NQB, C::NW, C::DQ_BN, kGeneral, 1, true>),
                        dim3((unsigned)((a.T + BM - 1) / BM) * BH), dim3(C::NW * 64), 0, st, a);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    const int n_scale = a.per_head_scale ? a.H : 1, n_tau = a.per_head_tau ? a.H : 1;
-    hipLaunchKernelGGL(purified_param_reduce_kernel<0>, dim3((unsigned)(n_scale + n_tau)), dim3(256), 0, st, a, nwg,
-                       n_scale);
-    return hipGetLastError();
+    return launch_purified_param_reduce(a, nwg, st);
 }
 
 template <class E>

@@ -160,7 +160,42 @@ def _stream_ptr(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
-def _check_inputs(q, k, v, scale_flat, doc_ids):
+def _run_call(fn, what: str, device: torch.device, block: bytes) -> None:
+    """One library call on ``device`` and its current stream.  The raw stream
+    handle and the device guard only where it is another device's turn: the
+    ``torch.cuda.Stream`` object and the guard cost more than the call."""
+    index = device.index
+    if torch.cuda.current_device() == index:
+        rc = fn(block, torch._C._cuda_getCurrentRawStream(index))
+    else:
+        with torch.cuda.device(device):
+            rc = fn(block, torch._C._cuda_getCurrentRawStream(index))
+    if rc != 0:
+        _native.check(rc, what)
+
+
+def _cast(t: torch.Tensor, dtype: torch.dtype, dp: int) -> torch.Tensor:
+    """``t`` in the compute dtype, zero-padded to ``dp`` columns, contiguous
+    and 16-byte aligned: itself where it already is."""
+    if t.dtype != dtype:
+        t = t.to(dtype)
+    return _aligned(_pad_head(t, dp))
+
+
+def _parameter(x, device: torch.device):
+    """A scale or tau for the argument block: (fp32 device tensor or None,
+    address, count, value).  A plain number travels by value: no device copy,
+    and no synchronisation with the device."""
+    if not isinstance(x, torch.Tensor):
+        return None, 0, 1, float(x)
+    flat = x.detach().contiguous()
+    if flat.dtype != torch.float32 or flat.device != device:
+        flat = flat.to(dtype=torch.float32, device=device)
+    return flat, flat.data_ptr(), flat.numel(), 0.0
+
+
+def _check_inputs(q, k, v, scale, doc_ids):
+    """Shapes of a call; ``scale``: its values, or how many there are."""
     if q.dim() != 4:
         raise ValueError(f"q must be (B, H, T, D), got shape {tuple(q.shape)}")
     if k.shape != q.shape or v.shape != q.shape:
@@ -171,7 +206,7 @@ def _check_inputs(q, k, v, scale_flat, doc_ids):
     B, H, T, D = q.shape
     if D > MAX_HEAD_DIM:
         raise NotImplementedError(f"head_dim {D} > {MAX_HEAD_DIM} is not supported by the HIP kernels")
-    n = scale_flat.numel()
+    n = scale if isinstance(scale, int) else scale.numel()
     if n not in (1, H):
         raise ValueError(f"scale must hold 1 value or H={H} per-head values, got {n}")
     if doc_ids is not None and tuple(doc_ids.shape) != (B, T):
@@ -194,7 +229,7 @@ class _FlashBornAttentionFn(torch.autograd.Function):
         q: torch.Tensor,
         k: torch.Tensor,
         v: torch.Tensor,
-        scale: torch.Tensor,
+        scale: float | torch.Tensor,
         is_causal: bool,
         eps: float,
         window_size: int = 0,
@@ -204,43 +239,31 @@ class _FlashBornAttentionFn(torch.autograd.Function):
         target = _autocast_dtype(q) or v.dtype
         if target not in _DTYPE_CODE:
             raise TypeError(f"flash_born_attention: unsupported dtype {target}")
-        scale_flat = scale.detach().contiguous().view(-1).to(dtype=torch.float32, device=q.device)
-        _check_inputs(q, k, v, scale_flat, doc_ids)
+        dev = q.device
+        scale_flat, scale_p, n_scale, scale_value = _parameter(scale, dev)
+        _check_inputs(q, k, v, n_scale, doc_ids)
         B, H, T, D = q.shape
         dp = (D + 7) // 8 * 8
-        q_c = _aligned(_pad_head(q.to(target), dp))
-        k_c = _aligned(_pad_head(k.to(target), dp))
-        v_c = _aligned(_pad_head(v.to(target), dp))
-        if doc_ids is not None:
-            doc_c = _aligned(doc_ids.to(device=q.device, dtype=torch.int32))
-        else:
-            doc_c = torch.empty(0, device=q.device, dtype=torch.int32)
+        q_c, k_c, v_c = _cast(q, target, dp), _cast(k, target, dp), _cast(v, target, dp)
+        doc_c = None if doc_ids is None else _aligned(doc_ids.to(device=dev, dtype=torch.int32))
         out = torch.empty_like(q_c)
-        z = torch.empty((B, H, T), dtype=torch.float32, device=q.device)
-        window = int(window_size)
-        if window < 0:
-            window = 0
-        with torch.cuda.device(q.device):
-            rc = lib.qdl_flash_born_fwd(
-                _DTYPE_CODE[target], B, H, T, dp,
-                q_c.data_ptr(), k_c.data_ptr(), v_c.data_ptr(), out.data_ptr(), z.data_ptr(),
-                scale_flat.data_ptr(), scale_flat.numel(),
-                doc_c.data_ptr() if doc_ids is not None else None,
-                1 if is_causal else 0, window, float(eps), _stream_ptr(q.device),
-            )
-        _native.check(rc, "qdl_flash_born_fwd")
+        z = torch.empty((B, H, T), dtype=torch.float32, device=dev)
+        window = max(int(window_size), 0)
+        _run_call(lib.qdl_flash_born_forward_call, "qdl_flash_born_forward_call", dev, _native.pack_call(
+            _DTYPE_CODE[target], B, H, T, dp,
+            q_c.data_ptr(), k_c.data_ptr(), v_c.data_ptr(), out.data_ptr(), z.data_ptr(),
+            scale_p, n_scale, scale_value, 0 if doc_c is None else doc_c.data_ptr(),
+            1 if is_causal else 0, window, float(eps)))
 
         ctx.save_for_backward(q_c, k_c, v_c, out, z, scale_flat, doc_c)
         ctx.is_causal = bool(is_causal)
         ctx.window_size = window
         ctx.eps = float(eps)
-        ctx.has_doc_ids = doc_ids is not None
         ctx.head_dim = D
-        ctx.scale_shape = scale.shape
-        ctx.scale_dtype = scale.dtype
-        ctx.orig_q_dtype = q.dtype
-        ctx.orig_k_dtype = k.dtype
-        ctx.orig_v_dtype = v.dtype
+        ctx.scale_value = scale_value
+        if scale_flat is not None:
+            ctx.scale_shape, ctx.scale_dtype = scale.shape, scale.dtype
+        ctx.dtypes = (q.dtype, k.dtype, v.dtype)
         return out if dp == D else out[..., :D].contiguous()
 
     @staticmethod
@@ -249,47 +272,57 @@ class _FlashBornAttentionFn(torch.autograd.Function):
         q_c, k_c, v_c, out, z, scale_flat, doc_c = ctx.saved_tensors
         B, H, T, dp = q_c.shape
         D = ctx.head_dim
-        do_c = _aligned(_pad_head(do.to(v_c.dtype), dp))
+        dev = q_c.device
+        do_c = _cast(do, v_c.dtype, dp)
         dq = torch.empty_like(q_c)
         dk = torch.empty_like(k_c)
         dv = torch.empty_like(v_c)
-        dscale = torch.empty(scale_flat.numel(), dtype=torch.float32, device=q_c.device)
+        n_scale = 1 if scale_flat is None else scale_flat.numel()
+        # The scale's gradient costs launches of its own: only where wanted.
+        dscale = torch.empty(n_scale, dtype=torch.float32, device=dev) if ctx.needs_input_grad[3] else None
         code = _DTYPE_CODE[v_c.dtype]
-        ws_bytes = int(lib.qdl_flash_born_bwd_workspace_size(code, B, H, T, dp, scale_flat.numel()))
-        ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=q_c.device)
-        with torch.cuda.device(q_c.device):
-            rc = lib.qdl_flash_born_bwd(
-                code, B, H, T, dp,
-                q_c.data_ptr(), k_c.data_ptr(), v_c.data_ptr(), out.data_ptr(), do_c.data_ptr(),
-                z.data_ptr(), scale_flat.data_ptr(), scale_flat.numel(),
-                doc_c.data_ptr() if ctx.has_doc_ids else None,
-                1 if ctx.is_causal else 0, ctx.window_size, ctx.eps,
-                dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dscale.data_ptr(),
-                ws.data_ptr(), ws.numel(), _stream_ptr(q_c.device),
-            )
-        _native.check(rc, "qdl_flash_born_bwd")
+        ws_bytes = int(lib.qdl_flash_born_bwd_workspace_size(code, B, H, T, dp, n_scale))
+        ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=dev)
+        _run_call(lib.qdl_flash_born_backward_call, "qdl_flash_born_backward_call", dev, _native.pack_call(
+            code, B, H, T, dp,
+            q_c.data_ptr(), k_c.data_ptr(), v_c.data_ptr(), out.data_ptr(), z.data_ptr(),
+            0 if scale_flat is None else scale_flat.data_ptr(), n_scale, ctx.scale_value,
+            0 if doc_c is None else doc_c.data_ptr(), 1 if ctx.is_causal else 0, ctx.window_size, ctx.eps,
+            dout=do_c.data_ptr(), dq=dq.data_ptr(), dk=dk.data_ptr(), dv=dv.data_ptr(),
+            dscale=0 if dscale is None else dscale.data_ptr(),
+            workspace=ws.data_ptr(), workspace_bytes=ws_bytes))
         if dp != D:
             dq, dk, dv = dq[..., :D], dk[..., :D], dv[..., :D]
-        dq_out = dq.to(ctx.orig_q_dtype)
-        dk_out = dk.to(ctx.orig_k_dtype)
-        dv_out = dv.to(ctx.orig_v_dtype)
-        dscale_out = dscale.view(ctx.scale_shape).to(ctx.scale_dtype)
-        return dq_out, dk_out, dv_out, dscale_out, None, None, None, None
+        qd, kd, vd = ctx.dtypes
+        return (dq.to(qd), dk.to(kd), dv.to(vd),
+                None if dscale is None else dscale.view(ctx.scale_shape).to(ctx.scale_dtype),
+                None, None, None, None)
 
 
+# A graph break under torch.compile (the reference's @torch.compiler.disable,
+# flash_born.py:620); outside of it the decorator's wrapper costs several
+# microseconds a call, so it is entered only while a compiler traces.
 @torch.compiler.disable
+def _apply_uncompiled(fn, args):
+    return fn.apply(*args)
+
+
+def _apply(fn, *args):
+    return _apply_uncompiled(fn, args) if torch.compiler.is_compiling() else fn.apply(*args)
+
+
 def _run_triton_flash_born(
     q: torch.Tensor,
     k: torch.Tensor,
     v: torch.Tensor,
-    scale_t: torch.Tensor,
+    scale_t: float | torch.Tensor,
     is_causal: bool,
     eps: float,
     window_size: int = 0,
     doc_ids: torch.Tensor | None = None,
 ) -> torch.Tensor:
     """Direct entry to the GPU kernels (reference name, flash_born.py:621-632)."""
-    return _FlashBornAttentionFn.apply(q, k, v, scale_t, is_causal, eps, int(window_size), doc_ids)
+    return _apply(_FlashBornAttentionFn, q, k, v, scale_t, is_causal, eps, int(window_size), doc_ids)
 
 
 _run_hip_flash_born = _run_triton_flash_born
@@ -346,12 +379,9 @@ def flash_born_attention(
     kernels for any head dim up to 256; CPU tensors and larger head dims use
     the eager formulation.
     """
-    if not isinstance(scale, torch.Tensor):
-        scale_t = torch.tensor(float(scale), dtype=torch.float32, device=q.device)
-    else:
-        scale_t = scale
     if q.is_cuda and q.shape[-1] <= MAX_HEAD_DIM:
-        return _run_triton_flash_born(q, k, v, scale_t, is_causal, eps, window_size=window_size, doc_ids=doc_ids)
+        return _run_triton_flash_born(q, k, v, scale, is_causal, eps, window_size=window_size, doc_ids=doc_ids)
+    scale_t = scale if isinstance(scale, torch.Tensor) else torch.tensor(float(scale), dtype=torch.float32, device=q.device)
     # CPU tensors, and head dims the kernels do not take (D > 256), run the
     # reference's eager formulation on the tensors' own device, as the
     # reference does for every shape its kernel does not support
@@ -380,8 +410,8 @@ class _FlashPurifiedBornAttentionFn(torch.autograd.Function):
         q: torch.Tensor,
         k: torch.Tensor,
         v: torch.Tensor,
-        scale: torch.Tensor,
-        tau: torch.Tensor,
+        scale: float | torch.Tensor,
+        tau: float | torch.Tensor,
         eps_base: float,
         is_causal: bool,
         eps: float,
@@ -392,41 +422,33 @@ class _FlashPurifiedBornAttentionFn(torch.autograd.Function):
         target = _autocast_dtype(q) or v.dtype
         if target not in _DTYPE_CODE:
             raise TypeError(f"flash_purified_born_attention: unsupported dtype {target}")
-        scale_flat = scale.detach().contiguous().view(-1).to(dtype=torch.float32, device=q.device)
-        tau_flat = tau.detach().contiguous().view(-1).to(dtype=torch.float32, device=q.device)
-        _check_inputs(q, k, v, scale_flat, doc_ids)
+        dev = q.device
+        scale_flat, scale_p, n_scale, scale_value = _parameter(scale, dev)
+        tau_flat, tau_p, n_tau, tau_value = _parameter(tau, dev)
+        _check_inputs(q, k, v, n_scale, doc_ids)
         B, H, T, D = q.shape
-        if tau_flat.numel() not in (1, H):
-            raise ValueError(f"tau must hold 1 value or H={H} per-head values, got {tau_flat.numel()}")
+        if n_tau not in (1, H):
+            raise ValueError(f"tau must hold 1 value or H={H} per-head values, got {n_tau}")
         dp = (D + 7) // 8 * 8
-        q_c = _aligned(_pad_head(q.to(target), dp))
-        k_c = _aligned(_pad_head(k.to(target), dp))
-        v_c = _aligned(_pad_head(v.to(target), dp))
-        if doc_ids is not None:
-            doc_c = _aligned(doc_ids.to(device=q.device, dtype=torch.int32))
-        else:
-            doc_c = torch.empty(0, device=q.device, dtype=torch.int32)
-        out_f32 = torch.empty((B, H, T, dp), dtype=torch.float32, device=q.device)
-        z = torch.empty((B, H, T), dtype=torch.float32, device=q.device)
+        q_c, k_c, v_c = _cast(q, target, dp), _cast(k, target, dp), _cast(v, target, dp)
+        doc_c = None if doc_ids is None else _aligned(doc_ids.to(device=dev, dtype=torch.int32))
+        out_f32 = torch.empty((B, H, T, dp), dtype=torch.float32, device=dev)
+        z = torch.empty((B, H, T), dtype=torch.float32, device=dev)
         window = max(int(window_size), 0)
-        with torch.cuda.device(q.device):
-            rc = lib.qdl_flash_purified_born_fwd(
-                _DTYPE_CODE[target], B, H, T, dp,
-                q_c.data_ptr(), k_c.data_ptr(), v_c.data_ptr(), out_f32.data_ptr(), z.data_ptr(),
-                scale_flat.data_ptr(), scale_flat.numel(), tau_flat.data_ptr(), tau_flat.numel(),
-                float(eps_base), doc_c.data_ptr() if doc_ids is not None else None,
-                1 if is_causal else 0, window, float(eps), _stream_ptr(q.device),
-            )
-        _native.check(rc, "qdl_flash_purified_born_fwd")
+        _run_call(lib.qdl_flash_born_forward_call, "qdl_flash_born_forward_call (purified)", dev, _native.pack_call(
+            _DTYPE_CODE[target], B, H, T, dp,
+            q_c.data_ptr(), k_c.data_ptr(), v_c.data_ptr(), out_f32.data_ptr(), z.data_ptr(),
+            scale_p, n_scale, scale_value, 0 if doc_c is None else doc_c.data_ptr(),
+            1 if is_causal else 0, window, float(eps),
+            purified=1, tau=tau_p, n_tau=n_tau, tau_value=tau_value, eps_base=float(eps_base)))
         ctx.save_for_backward(q_c, k_c, v_c, out_f32, z, scale_flat, tau_flat, doc_c)
         ctx.is_causal = bool(is_causal)
         ctx.window_size = window
         ctx.eps_base = float(eps_base)
-        ctx.has_doc_ids = doc_ids is not None
         ctx.head_dim = D
-        ctx.scale_shape, ctx.scale_dtype = scale.shape, scale.dtype
-        ctx.tau_shape, ctx.tau_dtype = tau.shape, tau.dtype
-        ctx.orig_q_dtype, ctx.orig_k_dtype, ctx.orig_v_dtype = q.dtype, k.dtype, v.dtype
+        ctx.values = (scale_value, tau_value)
+        ctx.shapes = tuple((p.shape, p.dtype) if isinstance(p, torch.Tensor) else None for p in (scale, tau))
+        ctx.dtypes = (q.dtype, k.dtype, v.dtype)
         out = out_f32 if dp == D else out_f32[..., :D]
         return out.to(target)
 
@@ -436,49 +458,42 @@ class _FlashPurifiedBornAttentionFn(torch.autograd.Function):
         q_c, k_c, v_c, out_f32, z, scale_flat, tau_flat, doc_c = ctx.saved_tensors
         B, H, T, dp = q_c.shape
         D = ctx.head_dim
-        do_c = _aligned(_pad_head(do.to(v_c.dtype), dp))
+        dev = q_c.device
+        do_c = _cast(do, v_c.dtype, dp)
         dq = torch.empty_like(q_c)
         dk = torch.empty_like(k_c)
         dv = torch.empty_like(v_c)
-        dscale = torch.empty(scale_flat.numel(), dtype=torch.float32, device=q_c.device)
-        dtau = torch.empty(tau_flat.numel(), dtype=torch.float32, device=q_c.device)
+        n_scale = 1 if scale_flat is None else scale_flat.numel()
+        n_tau = 1 if tau_flat is None else tau_flat.numel()
+        want_scale, want_tau = ctx.needs_input_grad[3], ctx.needs_input_grad[4]
+        dscale = torch.empty(n_scale, dtype=torch.float32, device=dev) if want_scale else None
+        dtau = torch.empty(n_tau, dtype=torch.float32, device=dev) if want_tau else None
         code = _DTYPE_CODE[v_c.dtype]
         ws_bytes = int(lib.qdl_flash_purified_born_bwd_workspace_size(code, B, H, T, dp))
-        ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=q_c.device)
-        with torch.cuda.device(q_c.device):
-            rc = lib.qdl_flash_purified_born_bwd(
-                code, B, H, T, dp,
-                q_c.data_ptr(), k_c.data_ptr(), v_c.data_ptr(), out_f32.data_ptr(), do_c.data_ptr(),
-                z.data_ptr(), scale_flat.data_ptr(), scale_flat.numel(), tau_flat.data_ptr(), tau_flat.numel(),
-                ctx.eps_base, doc_c.data_ptr() if ctx.has_doc_ids else None,
-                1 if ctx.is_causal else 0, ctx.window_size,
-                dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dscale.data_ptr(), dtau.data_ptr(),
-                ws.data_ptr(), ws.numel(), _stream_ptr(q_c.device),
-            )
-        _native.check(rc, "qdl_flash_purified_born_bwd")
+        ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=dev)
+        scale_value, tau_value = ctx.values
+        _run_call(lib.qdl_flash_born_backward_call, "qdl_flash_born_backward_call (purified)", dev, _native.pack_call(
+            code, B, H, T, dp,
+            q_c.data_ptr(), k_c.data_ptr(), v_c.data_ptr(), out_f32.data_ptr(), z.data_ptr(),
+            0 if scale_flat is None else scale_flat.data_ptr(), n_scale, scale_value,
+            0 if doc_c is None else doc_c.data_ptr(), 1 if ctx.is_causal else 0, ctx.window_size, 0.0,
+            purified=1, tau=0 if tau_flat is None else tau_flat.data_ptr(), n_tau=n_tau, tau_value=tau_value,
+            eps_base=ctx.eps_base, dout=do_c.data_ptr(), dq=dq.data_ptr(), dk=dk.data_ptr(), dv=dv.data_ptr(),
+            dscale=0 if dscale is None else dscale.data_ptr(), dtau=0 if dtau is None else dtau.data_ptr(),
+            workspace=ws.data_ptr(), workspace_bytes=ws_bytes))
         if dp != D:
             dq, dk, dv = dq[..., :D], dk[..., :D], dv[..., :D]
-        return (
-            dq.to(ctx.orig_q_dtype),
-            dk.to(ctx.orig_k_dtype),
-            dv.to(ctx.orig_v_dtype),
-            dscale.view(ctx.scale_shape).to(ctx.scale_dtype),
-            dtau.view(ctx.tau_shape).to(ctx.tau_dtype),
-            None,
-            None,
-            None,
-            None,
-            None,
-        )
+        qd, kd, vd = ctx.dtypes
+        params = (None if g is None else g.view(sd[0]).to(sd[1]) for g, sd in zip((dscale, dtau), ctx.shapes))
+        return (dq.to(qd), dk.to(kd), dv.to(vd), *params, None, None, None, None, None)
 
 
-@torch.compiler.disable
 def _run_triton_flash_purified_born(
     q: torch.Tensor,
     k: torch.Tensor,
     v: torch.Tensor,
-    scale_t: torch.Tensor,
-    tau_t: torch.Tensor,
+    scale_t: float | torch.Tensor,
+    tau_t: float | torch.Tensor,
     eps_base: float,
     is_causal: bool,
     eps: float,
@@ -486,8 +501,8 @@ def _run_triton_flash_purified_born(
     doc_ids: torch.Tensor | None = None,
 ) -> torch.Tensor:
     """Direct entry to the GPU kernels (reference name, flash_born.py:1273-1287)."""
-    return _FlashPurifiedBornAttentionFn.apply(
-        q, k, v, scale_t, tau_t, eps_base, is_causal, eps, int(window_size), doc_ids
+    return _apply(
+        _FlashPurifiedBornAttentionFn, q, k, v, scale_t, tau_t, eps_base, is_causal, eps, int(window_size), doc_ids
     )
 
 
@@ -543,12 +558,12 @@ def flash_purified_born_attention(
         tau = tau_h if tau_h is not None else 0.0625
     if causal is not None:
         is_causal = bool(causal)
-    scale_t = scale if isinstance(scale, torch.Tensor) else torch.tensor(float(scale), dtype=torch.float32, device=q.device)
-    tau_t = tau if isinstance(tau, torch.Tensor) else torch.tensor(float(tau), dtype=torch.float32, device=q.device)
     if q.is_cuda and q.shape[-1] <= MAX_HEAD_DIM:
         return _run_triton_flash_purified_born(
-            q, k, v, scale_t, tau_t, eps_base, is_causal, eps, window_size=window_size, doc_ids=doc_ids
+            q, k, v, scale, tau, eps_base, is_causal, eps, window_size=window_size, doc_ids=doc_ids
         )
+    scale_t, tau_t = (x if isinstance(x, torch.Tensor) else torch.tensor(float(x), dtype=torch.float32, device=q.device)
+                      for x in (scale, tau))
     # CPU tensors and D > 256: the reference's eager formulation on the
     # tensors' own device (flash_born.py:1318-1341).
     return _eager_purified_born(q, k, v, scale_t, tau_t, eps_base, is_causal, eps, window_size, doc_ids)

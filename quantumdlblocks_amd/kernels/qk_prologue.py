@@ -124,49 +124,16 @@ def _dense_layout(shape, strides) -> bool:
     return True
 
 
-def _launch_bwd(g, out, rinv, cos2, sin2, layout, which: int):
-    """Input gradient of one tensor, written with the input's (shape, strides)
-    when those are dense (a permuted contiguous tensor, e.g. the projection
-    layout) with unit stride along D, else contiguous.  The kernel writes each
-    D row contiguously and takes only the (b, h, t) strides, so an input whose
-    D stride is not 1 (e.g. a transposed (B, H, D, T) tensor) gets a
-    contiguous gradient."""
-    lib = _native.load()
-    B, H, T, D = out.shape
-    g = g.to(out.dtype).contiguous()
-    shape, strides = layout
-    if _dense_layout(shape, strides) and (shape[-1] == 1 or strides[-1] == 1):
-        dx = torch.empty_strided(layout[0], layout[1], dtype=out.dtype, device=out.device)
-    else:
-        dx = torch.empty(layout[0], dtype=out.dtype, device=out.device)
-    st = _strides(dx)
-    gs = [None, None]
-    ys = [None, None]
-    rs = [None, None]
-    ds = [None, None, None, None]
-    gs[which] = g.data_ptr()
-    ys[which] = out.data_ptr()
-    rs[which] = rinv.data_ptr()
-    ds[2 * which] = dx.data_ptr()
-    ds[2 * which + 1] = st.data_ptr()
-    with torch.cuda.device(out.device):
-        rc = lib.qdl_flash_born_qk_prologue_bwd(
-            _DTYPE_CODE[out.dtype], B, H, T, D, *gs, *ys, *rs,
-            cos2.data_ptr() if cos2 is not None else None,
-            sin2.data_ptr() if sin2 is not None else None,
-            cos2.shape[1] if cos2 is not None else 0,
-            cos2.stride(0) if cos2 is not None else 0,
-            *ds, _stream_ptr(out.device),
-        )
-    _native.check(rc, "qdl_flash_born_qk_prologue_bwd")
-    return dx
-
-
 def _prep_tables(cos, sin, half: int, T: int, device):
     """fp32 (T, n) tables with n = min(width, half) and one row stride, or
     (None, None)."""
     if cos is None:
         return None, None
+    n = cos.size(-1)
+    if (n <= half and sin.shape == cos.shape and cos.numel() == T * n and cos.dim() >= 2 and cos.shape[-2] == T
+            and all(t.dtype == torch.float32 and t.device == device and t.is_contiguous() and not t.requires_grad
+                    for t in (cos, sin))):
+        return cos.view(T, n), sin.view(T, n)  # the usual tables: no copies, one view each
     # Columns past the table's width rotate by angle 0 inside the kernel (the
     # reference's padding, attention.py:577-582).
     n = min(cos.size(-1), half)
@@ -208,20 +175,58 @@ def qk_prologue_forward(q, k, cos=None, sin=None, eps: float = 1e-12):
     return q_out, k_out, q_r, k_r
 
 
+def _grad_like(layout, dtype, device) -> torch.Tensor:
+    """An input gradient with the input's (shape, strides) when those are dense
+    (a permuted contiguous tensor, e.g. the projection layout) with unit stride
+    along D, else contiguous.  The kernel writes each D row contiguously and
+    takes only the (b, h, t) strides, so an input whose D stride is not 1 (e.g.
+    a transposed (B, H, D, T) tensor) gets a contiguous gradient."""
+    shape, strides = layout
+    if _dense_layout(shape, strides) and (shape[-1] == 1 or strides[-1] == 1):
+        return torch.empty_strided(shape, strides, dtype=dtype, device=device)
+    return torch.empty(shape, dtype=dtype, device=device)
+
+
 def qk_prologue_backward(gq, gk, q_out, k_out, q_rinv, k_rinv, cos=None, sin=None,
                          q_layout=None, k_layout=None):
     """No-autograd backward: input gradients (None where the output gradient
     is None), written with ``(shape, strides)`` layouts (default contiguous)."""
     B, H, T, D = q_out.shape
     cos2, sin2 = _prep_tables(cos, sin, D // 2, T, q_out.device)
-    dq = dk = None
-    if gq is not None:
-        lay = q_layout or (tuple(q_out.shape), tuple(q_out.stride()))
-        dq = _launch_bwd(gq, q_out, q_rinv, cos2, sin2, lay, 0)
-    if gk is not None:
-        lay = k_layout or (tuple(k_out.shape), tuple(k_out.stride()))
-        dk = _launch_bwd(gk, k_out, k_rinv, cos2, sin2, lay, 1)
-    return dq, dk
+    jobs = []  # per tensor: (slot, output gradient, output, 1/norm, input gradient)
+    for which, (g, out, rinv, layout) in enumerate(((gq, q_out, q_rinv, q_layout), (gk, k_out, k_rinv, k_layout))):
+        if g is None:
+            continue
+        dx = _grad_like(layout or (tuple(out.shape), tuple(out.stride())), out.dtype, out.device)
+        jobs.append((which, g.to(out.dtype).contiguous(), out, rinv, dx))
+    # One launch for both, unless their dtypes or devices differ.
+    together = len({(j[2].dtype, j[2].device) for j in jobs}) <= 1
+    for batch in [jobs] if together and jobs else [[j] for j in jobs]:
+        _launch_bwd(batch, (B, H, T, D), cos2, sin2)
+    grads = {j[0]: j[4] for j in jobs}
+    return grads.get(0), grads.get(1)
+
+
+def _launch_bwd(jobs, shape, cos2, sin2) -> None:
+    """The prologue backward of one or both tensors of one dtype and device."""
+    lib = _native.load()
+    gs, ys, rs, ds, strides = [None] * 2, [None] * 2, [None] * 2, [None] * 4, []
+    for which, g, out, rinv, dx in jobs:
+        st = _strides(dx)
+        strides.append(st)  # alive until the call
+        gs[which], ys[which], rs[which] = g.data_ptr(), out.data_ptr(), rinv.data_ptr()
+        ds[2 * which], ds[2 * which + 1] = dx.data_ptr(), st.data_ptr()
+    out = jobs[0][2]
+    with torch.cuda.device(out.device):
+        rc = lib.qdl_flash_born_qk_prologue_bwd(
+            _DTYPE_CODE[out.dtype], *shape, *gs, *ys, *rs,
+            cos2.data_ptr() if cos2 is not None else None,
+            sin2.data_ptr() if sin2 is not None else None,
+            cos2.shape[1] if cos2 is not None else 0,
+            cos2.stride(0) if cos2 is not None else 0,
+            *ds, _stream_ptr(out.device),
+        )
+    _native.check(rc, "qdl_flash_born_qk_prologue_bwd")
 
 
 class _QKPrologueFn(torch.autograd.Function):
@@ -298,54 +303,48 @@ class _BornQKPrologueFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, v, scale, cos, sin, is_causal, eps, window_size, doc_ids, norm_eps):
-        from .flash_born import _aligned, _autocast_dtype, _check_inputs
+        from .flash_born import _aligned, _autocast_dtype, _check_inputs, _parameter, _run_call
 
         lib = _native.load()
         target = _autocast_dtype(q) or v.dtype
         if target not in _DTYPE_CODE:
             raise TypeError(f"flash_born_attention_qk_prologue: unsupported dtype {target}")
-        scale_flat = scale.detach().contiguous().view(-1).to(dtype=torch.float32, device=q.device)
-        _check_inputs(q, k, v, scale_flat, doc_ids)
+        dev = q.device
+        scale_flat, scale_p, n_scale, scale_value = _parameter(scale, dev)
+        _check_inputs(q, k, v, n_scale, doc_ids)
         B, H, T, D = q.shape
         q_in = _rows_ok(q.detach().to(target))
         k_in = _rows_ok(k.detach().to(target))
         v_c = _aligned(v.detach().to(target))
-        cos2, sin2 = _prep_tables(cos, sin, D // 2, T, q.device)
-        doc_c = None if doc_ids is None else _aligned(doc_ids.to(device=q.device, dtype=torch.int32))
-        out = torch.empty((B, H, T, D), dtype=target, device=q.device)
-        z = torch.empty((B, H, T), dtype=torch.float32, device=q.device)
+        cos2, sin2 = _prep_tables(cos, sin, D // 2, T, dev)
+        doc_c = None if doc_ids is None else _aligned(doc_ids.to(device=dev, dtype=torch.int32))
+        out = torch.empty((B, H, T, D), dtype=target, device=dev)
+        z = torch.empty((B, H, T), dtype=torch.float32, device=dev)
         q_out = torch.empty_like(out)
         k_out = torch.empty_like(out)
         grad = any(ctx.needs_input_grad[:4])
         q_r = torch.empty_like(z) if grad else None
         k_r = torch.empty_like(z) if grad else None
-        qs, ks = _strides(q_in), _strides(k_in)
         window = max(int(window_size), 0)
-        with torch.cuda.device(q.device):
-            rc = lib.qdl_flash_born_fwd_qk_prologue(
-                _DTYPE_CODE[target], B, H, T, D,
-                q_in.data_ptr(), qs.data_ptr(), k_in.data_ptr(), ks.data_ptr(), v_c.data_ptr(),
-                cos2.data_ptr() if cos2 is not None else None,
-                sin2.data_ptr() if sin2 is not None else None,
-                cos2.shape[1] if cos2 is not None else 0,
-                cos2.stride(0) if cos2 is not None else 0,
-                float(norm_eps), scale_flat.data_ptr(), scale_flat.numel(),
-                doc_c.data_ptr() if doc_c is not None else None,
-                1 if is_causal else 0, window, float(eps),
-                out.data_ptr(), z.data_ptr(), q_out.data_ptr(), k_out.data_ptr(),
-                q_r.data_ptr() if grad else None, k_r.data_ptr() if grad else None, _stream_ptr(q.device),
-            )
-        _native.check(rc, "qdl_flash_born_fwd_qk_prologue")
+        tables = (0, 0, 0, 0) if cos2 is None else (cos2.data_ptr(), sin2.data_ptr(), cos2.shape[1], cos2.stride(0))
+        _run_call(lib.qdl_flash_born_forward_call, "qdl_flash_born_forward_call (prologue)", dev, _native.pack_call(
+            _DTYPE_CODE[target], B, H, T, D,
+            q_in.data_ptr(), k_in.data_ptr(), v_c.data_ptr(), out.data_ptr(), z.data_ptr(),
+            scale_p, n_scale, scale_value, 0 if doc_c is None else doc_c.data_ptr(),
+            1 if is_causal else 0, window, float(eps),
+            prologue=(1, *q_in.stride()[:3], *k_in.stride()[:3], *tables, float(norm_eps),
+                      q_out.data_ptr(), k_out.data_ptr(),
+                      q_r.data_ptr() if grad else 0, k_r.data_ptr() if grad else 0)))
         if not grad:
             return out
-        ctx.save_for_backward(q_out, k_out, v_c, out, z, scale_flat, q_r, k_r,
-                              doc_c if doc_c is not None else torch.empty(0, dtype=torch.int32, device=q.device))
+        ctx.save_for_backward(q_out, k_out, v_c, out, z, scale_flat, q_r, k_r, doc_c)
         ctx.tables = (cos.detach(), sin.detach()) if cos is not None else (None, None)
         ctx.q_layout = (tuple(q.shape), tuple(q.stride()))
         ctx.k_layout = (tuple(k.shape), tuple(k.stride()))
         ctx.is_causal, ctx.eps, ctx.window_size = bool(is_causal), float(eps), window
-        ctx.has_doc_ids = doc_ids is not None
-        ctx.scale_shape, ctx.scale_dtype = scale.shape, scale.dtype
+        ctx.scale_value = scale_value
+        if scale_flat is not None:
+            ctx.scale_shape, ctx.scale_dtype = scale.shape, scale.dtype
         ctx.dtypes = (q.dtype, k.dtype, v.dtype)
         return out
 
@@ -354,31 +353,31 @@ class _BornQKPrologueFn(torch.autograd.Function):
         lib = _native.load()
         q_out, k_out, v_c, out, z, scale_flat, q_r, k_r, doc_c = ctx.saved_tensors
         B, H, T, D = q_out.shape
-        from .flash_born import _aligned
+        dev = q_out.device
+        from .flash_born import _aligned, _run_call
 
         do_c = _aligned(do.to(v_c.dtype))
         dqn = torch.empty_like(q_out)
         dkn = torch.empty_like(k_out)
         dv = torch.empty_like(v_c)
-        dscale = torch.empty(scale_flat.numel(), dtype=torch.float32, device=q_out.device)
+        n_scale = 1 if scale_flat is None else scale_flat.numel()
+        dscale = torch.empty(n_scale, dtype=torch.float32, device=dev) if ctx.needs_input_grad[3] else None
         code = _DTYPE_CODE[v_c.dtype]
-        ws_bytes = int(lib.qdl_flash_born_bwd_workspace_size(code, B, H, T, D, scale_flat.numel()))
-        ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=q_out.device)
-        with torch.cuda.device(q_out.device):
-            rc = lib.qdl_flash_born_bwd(
-                code, B, H, T, D,
-                q_out.data_ptr(), k_out.data_ptr(), v_c.data_ptr(), out.data_ptr(), do_c.data_ptr(),
-                z.data_ptr(), scale_flat.data_ptr(), scale_flat.numel(),
-                doc_c.data_ptr() if ctx.has_doc_ids else None,
-                1 if ctx.is_causal else 0, ctx.window_size, ctx.eps,
-                dqn.data_ptr(), dkn.data_ptr(), dv.data_ptr(), dscale.data_ptr(),
-                ws.data_ptr(), ws.numel(), _stream_ptr(q_out.device),
-            )
-        _native.check(rc, "qdl_flash_born_bwd")
+        ws_bytes = int(lib.qdl_flash_born_bwd_workspace_size(code, B, H, T, D, n_scale))
+        ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=dev)
+        _run_call(lib.qdl_flash_born_backward_call, "qdl_flash_born_backward_call", dev, _native.pack_call(
+            code, B, H, T, D,
+            q_out.data_ptr(), k_out.data_ptr(), v_c.data_ptr(), out.data_ptr(), z.data_ptr(),
+            0 if scale_flat is None else scale_flat.data_ptr(), n_scale, ctx.scale_value,
+            0 if doc_c is None else doc_c.data_ptr(), 1 if ctx.is_causal else 0, ctx.window_size, ctx.eps,
+            dout=do_c.data_ptr(), dq=dqn.data_ptr(), dk=dkn.data_ptr(), dv=dv.data_ptr(),
+            dscale=0 if dscale is None else dscale.data_ptr(),
+            workspace=ws.data_ptr(), workspace_bytes=ws_bytes))
         cos, sin = ctx.tables
         dq, dk = qk_prologue_backward(dqn, dkn, q_out, k_out, q_r, k_r, cos, sin, ctx.q_layout, ctx.k_layout)
         qd, kd, vd = ctx.dtypes
-        return (dq.to(qd), dk.to(kd), dv.to(vd), dscale.view(ctx.scale_shape).to(ctx.scale_dtype),
+        return (dq.to(qd), dk.to(kd), dv.to(vd),
+                None if dscale is None else dscale.view(ctx.scale_shape).to(ctx.scale_dtype),
                 None, None, None, None, None, None, None)
 
 
@@ -414,8 +413,6 @@ def flash_born_attention_qk_prologue(
         raise ValueError("q, k, v must share one (B, H, T, D) shape")
     if (cos is None) != (sin is None):
         raise ValueError("cos and sin must be given together")
-    if not isinstance(scale, torch.Tensor):
-        scale = torch.tensor(float(scale), dtype=torch.float32, device=q.device)
     D = q.shape[-1]
     if not q.is_cuda or D % 8 or D > MAX_HEAD_DIM:
         qn, kn = fused_qk_rope_l2_normalize(q, k, cos, sin, norm_eps)

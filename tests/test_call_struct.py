@@ -1,0 +1,114 @@
+"""The struct-form entry points (qdl_flash_born_forward_call / _backward_call):
+the packed block matches the C struct, is validated before any launch, and a
+scale or tau passed by value gives what the same value in device memory does."""
+
+from __future__ import annotations
+
+import ctypes
+import os
+import re
+
+import pytest
+import torch
+
+HEADER = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "include", "qdl_flash_born.h")
+
+
+def _block(**kw):
+    from quantumdlblocks_amd import _native
+
+    args = dict(dtype=_native.DTYPE_BF16, B=1, H=2, T=8, D=64, q=0, k=0, v=0, out=0, z=0, scale=0, n_scale=1,
+                scale_value=8.0, doc=0, causal=1, window=0, eps=1e-12)
+    args.update(kw)
+    return _native.pack_call(**args)
+
+
+def test_block_has_the_structs_size():
+    body = re.search(r"typedef struct qdl_born_call \{(.*?)\} qdl_born_call;", open(HEADER).read(), re.S).group(1)
+    body = re.sub(r"/\*.*?\*/", "", body, flags=re.S)
+    fields = 0
+    for decl in body.split(";"):
+        for name in decl.split(",") if decl.strip() else []:
+            n = re.search(r"\[(\d+)\]", name)
+            fields += int(n.group(1)) if n else 1
+    assert len(_block()) == 8 * fields
+
+
+def test_validation():
+    from quantumdlblocks_amd import _native
+
+    lib = _native.load()
+    for fn in (lib.qdl_flash_born_forward_call, lib.qdl_flash_born_backward_call):
+        assert fn(None, None) == -5
+        assert fn(ctypes.c_char_p(b"\0" * 376), None) == -2  # struct_bytes
+        assert fn(_block(dtype=7), None) == -1
+        assert fn(_block(D=12), None) == -3
+        assert fn(_block(scale=64, n_scale=3), None) == -6
+        assert fn(_block(window=-1), None) == -7
+        assert fn(_block(purified=1, tau=64, n_tau=3), None) == -9
+        assert fn(_block(eps=-1.0), None) == -2
+        assert fn(_block(), None) == -5
+        assert fn(_block(T=0), None) == 0
+    ptrs = dict(q=16, k=16, v=16, out=16, z=16)
+    assert lib.qdl_flash_born_forward_call(_block(**{**ptrs, "q": 24}), None) == -4
+    assert lib.qdl_flash_born_backward_call(_block(**ptrs, dout=16, dq=16, dk=16, dv=16), None) == -8
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("purified", [False, True], ids=["born", "purified"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32], ids=str)
+@pytest.mark.parametrize("D", [40, 64, 100, 128, 200])
+@pytest.mark.parametrize("mask", [dict(), dict(is_causal=False), dict(window_size=30), dict(doc=True),
+                                  dict(is_causal=False, window_size=20, doc=True)], ids=str)
+def test_parameters_by_value(cuda_device, purified, dtype, D, mask):
+    """Every kernel reads scale and tau from the block or from memory: bitwise
+    the same output and gradients (no gradient of a plain number)."""
+    from quantumdlblocks_amd import flash_born_attention, flash_purified_born_attention
+
+    g = torch.Generator("cpu").manual_seed(D)
+    q, k, v, do = (torch.randn(1, 2, 70, D, generator=g).mul(0.3).to(cuda_device, dtype) for _ in range(4))
+    kw = dict(mask)
+    if kw.pop("doc", False):
+        kw["doc_ids"] = (torch.arange(70, device=cuda_device) // 25).view(1, 70)
+    got = []
+    for scale, tau in ((-1.5, 0.02), (torch.tensor([-1.5, -1.5], device=cuda_device, requires_grad=True),
+                                      torch.tensor(0.02, device=cuda_device))):
+        x = [t.clone().requires_grad_(True) for t in (q, k, v)]
+        if purified:
+            out = flash_purified_born_attention(*x, -scale, tau, **kw)
+        else:
+            out = flash_born_attention(*x, scale, **kw)
+        out.backward(do)
+        got.append([out, *(t.grad for t in x)])
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+def test_prologue_scale_by_value(cuda_device):
+    from quantumdlblocks_amd import flash_born_attention_qk_prologue
+
+    q, k, v = (torch.randn(2, 70, 4, 64, device=cuda_device, dtype=torch.bfloat16).transpose(1, 2) for _ in range(3))
+    a = flash_born_attention_qk_prologue(q, k, v, 3.0)
+    b = flash_born_attention_qk_prologue(q, k, v, torch.tensor(3.0, device=cuda_device))
+    assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+def test_a_call_captures_with_a_plain_scale(cuda_device):
+    """A float scale needs no copy from the host, so the call can be captured;
+    replays follow the inputs."""
+    from quantumdlblocks_amd import flash_born_attention
+
+    q, k, v = (torch.randn(1, 4, 96, 64, device=cuda_device, dtype=torch.bfloat16) for _ in range(3))
+    flash_born_attention(q, k, v, 2.0)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph), torch.no_grad():
+        out = flash_born_attention(q, k, v, 2.0)
+    for seed in range(3):
+        torch.manual_seed(seed)
+        q.copy_(torch.randn_like(q))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, flash_born_attention(q, k, v, 2.0))
