@@ -129,9 +129,9 @@ __device__ __forceinline__ void f32_issue_values(const void* v, int r0, int T, v
 // is resident at once, two workgroups per CU (257 to 512 of them), the second
 // half goes out shortest first, so that a CU pairs a long block with a short
 // one (B2 H8 T1000 D64 step: 159 -> 142 us).
-struct F32Block {
+struct SplitBlock {
     int bh, mb;
-    __device__ __forceinline__ F32Block(int bid, int grid, int BH, int nmb, bool longest_last) {
+    __device__ __forceinline__ SplitBlock(int bid, int grid, int BH, int nmb, bool longest_last) {
         const int rank = grid <= 512 && bid >= 256 ? grid - 1 - (bid - 256) : bid;
         bh = rank % BH;
         mb = longest_last ? nmb - 1 - rank / BH : rank / BH;
@@ -139,7 +139,7 @@ struct F32Block {
 };
 
 // Which (query, key) pairs a block's rows see.
-struct F32Mask {
+struct SplitMask {
     bool causal, has_doc;
     int window;
     __device__ __forceinline__ bool visible(int i, int j, int di, int dj) const {
@@ -208,8 +208,8 @@ void born_f32_fwd_kernel(typename std::conditional<PUR, PurArgs, FwdArgs>::type 
 
     const int T = p.T, D = p.D, BH = p.B * p.H;
     const int nmb = (T + kF32Rows - 1) / kF32Rows;
-    const F32Mask m = {p.is_causal != 0, p.doc != nullptr, p.window};
-    const F32Block blk((int)blockIdx.x, (int)gridDim.x, BH, nmb, m.causal);
+    const SplitMask m = {p.is_causal != 0, p.doc != nullptr, p.window};
+    const SplitBlock blk((int)blockIdx.x, (int)gridDim.x, BH, nmb, m.causal);
     const int b = blk.bh / p.H, h = blk.bh % p.H, m0 = blk.mb * kF32Rows;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -268,7 +268,8 @@ void born_f32_fwd_kernel(typename std::conditional<PUR, PurArgs, FwdArgs>::type 
 #pragma unroll
             for (int e = 0; e < 4; ++e) s = mfma_f32(a[e], qr[u][e], s);
         }
-        const int kdoc = m.has_doc && key0 + c < T ? kd_lds[wave][c] : -2;
+        int kdoc = m.has_doc && key0 + c < T ? kd_lds[wave][c] : -2;
+        asm volatile("" : "+v"(kdoc));  // read for good before the next ids are sent into its place
         __builtin_amdgcn_sched_barrier(0);
         if (more) issue_k(t + NW);
         bool cut = m.cuts(m0, key0) || (PUR && key0 + 32 > T);
@@ -366,8 +367,8 @@ void born_f32_dq_kernel(typename std::conditional<PUR, PurArgs, BwdArgs>::type p
 
     const int T = p.T, D = p.D, BH = p.B * p.H;
     const int nmb = (T + kF32Rows - 1) / kF32Rows;
-    const F32Mask m = {p.is_causal != 0, p.doc != nullptr, p.window};
-    const F32Block blk((int)blockIdx.x, (int)gridDim.x, BH, nmb, m.causal);
+    const SplitMask m = {p.is_causal != 0, p.doc != nullptr, p.window};
+    const SplitBlock blk((int)blockIdx.x, (int)gridDim.x, BH, nmb, m.causal);
     const int b = blk.bh / p.H, h = blk.bh % p.H, m0 = blk.mb * kF32Rows;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -457,7 +458,8 @@ void born_f32_dq_kernel(typename std::conditional<PUR, PurArgs, BwdArgs>::type p
 #pragma unroll
             for (int e = 0; e < 4; ++e) tt = mfma_f32(a[e], dr[u][e], tt);
         }
-        const int kdoc = m.has_doc && key0 + c < T ? kd_lds[wave][c] : -2;
+        int kdoc = m.has_doc && key0 + c < T ? kd_lds[wave][c] : -2;
+        asm volatile("" : "+v"(kdoc));  // read for good before the next ids are sent into its place
         __builtin_amdgcn_sched_barrier(0);
         if (more) {
             issue_v(t + NW);
@@ -535,8 +537,8 @@ void born_f32_dkdv_kernel(typename std::conditional<PUR, PurArgs, BwdArgs>::type
 
     const int T = p.T, D = p.D, BH = p.B * p.H;
     const int nkb = (T + kF32Rows - 1) / kF32Rows;
-    const F32Mask m = {p.is_causal != 0, p.doc != nullptr, p.window};
-    const F32Block blk((int)blockIdx.x, (int)gridDim.x, BH, nkb, false);
+    const SplitMask m = {p.is_causal != 0, p.doc != nullptr, p.window};
+    const SplitBlock blk((int)blockIdx.x, (int)gridDim.x, BH, nkb, false);
     const int b = blk.bh / p.H, h = blk.bh % p.H, k0 = blk.mb * kF32Rows;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
