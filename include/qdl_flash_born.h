@@ -191,6 +191,9 @@ int qdl_flash_purified_born_bwd(int dtype, int64_t B, int64_t H, int64_t T,
  *     that reduce it are left out;
  *   - purified != 0 selects the purified weights (out is then fp32), prologue
  *     != 0 the fused Q/K prologue (Born forward).
+ * param_grads keeps fp32 and fp16 purified calls whose scale or tau is trained
+ * on the kernels of the positional entry points: dscale is a cancelling sum,
+ * which the output's last bits (another summation order) move by up to 4e-3.
  * Other fields, results and return codes are those of the positional entry
  * points; struct_bytes must be sizeof(qdl_born_call) (else QDL_BORN_E_SHAPE).
  * Unused fields are ignored.
@@ -212,6 +215,7 @@ typedef struct qdl_born_call {
     int64_t n_tau;
     double tau_value;
     double eps_base;
+    int64_t param_grads; /* purified forward: != 0 if the backward will be asked for dscale or dtau */
     /* backward */
     const void *dout;
     void *dq, *dk, *dv;

@@ -45,6 +45,31 @@ __global__ __launch_bounds__(64) void born_bwd_dscale_final_kernel(BwdArgs p, co
     p.dscale[out] = (s == 0.f) ? 0.f : (float)(2.0 / (double)s * (double)p.eps * acc);
 }
 
+// The same sum in one launch, a workgroup per output: up to this many rows
+// each (64 loads per thread) it takes less than the second launch.
+constexpr int64_t kDscaleRows = 16384;
+__global__ __launch_bounds__(256) void born_bwd_dscale_rows_kernel(BwdArgs p) {
+    __shared__ double red[256];
+    const int out = blockIdx.x, tid = threadIdx.x;
+    const int n = p.per_head_scale ? p.B * p.T : p.B * p.H * p.T;
+    double acc = 0.0;
+#pragma unroll 8
+    for (int j = tid; j < n; j += 256) {
+        int idx = j;
+        if (p.per_head_scale) idx = (j / p.T * p.H + out) * p.T + j % p.T;
+        acc += (double)p.delta_z[idx];
+    }
+    red[tid] = acc;
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+        if (tid < w) red[tid] += red[tid + w];
+        __syncthreads();
+    }
+    if (tid != 0) return;
+    const float s = arg_scale(p, out);
+    p.dscale[out] = (s == 0.f) ? 0.f : (float)(2.0 / (double)s * (double)p.eps * red[0]);
+}
+
 __global__ void born_zero_fill_kernel(float* __restrict__ x, int64_t n) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
          i += (int64_t)gridDim.x * blockDim.x)
@@ -54,6 +79,10 @@ __global__ void born_zero_fill_kernel(float* __restrict__ x, int64_t n) {
 hipError_t launch_bwd_common_post(const BwdArgs& a, hipStream_t st) {
     if (a.dscale == nullptr) return hipSuccess;
     const int nout = a.per_head_scale ? a.H : 1;
+    if ((int64_t)a.B * a.H * a.T / nout <= kDscaleRows) {
+        hipLaunchKernelGGL(born_bwd_dscale_rows_kernel, dim3(nout), dim3(256), 0, st, a);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(born_bwd_dscale_partial_kernel, dim3(DSCALE_CHUNKS, nout), dim3(256), 0, st, a,
                        a.dscale_part);
     hipError_t e = hipGetLastError();

@@ -21,10 +21,6 @@ hipError_t bwd_launch_f32(const BwdArgs& a, hipStream_t s) {
     return hipErrorInvalidValue;
 }
 
-hipError_t purified_bwd_f32_launch(const PurArgs& a, hipStream_t s) {
-    const hipError_t e = launch_f32_bwd<true>(a, s);
-    if (e != hipSuccess) return e;
-    return launch_purified_param_reduce(a, f32_groups(a.B, a.H, a.T), s);
-}
+hipError_t purified_bwd_f32_launch(const PurArgs& a, hipStream_t s) { return launch_f32_bwd<true>(a, s); }
 
 }  // namespace qdl

@@ -90,6 +90,7 @@ int qdl_flash_born_forward_call(const qdl_born_call* c, qdl_stream_t stream) {
         fill_purified(a, c);
         a.o = static_cast<float*>(c->out);
         a.z = c->z;
+        a.param_grads = c->param_grads ? 1 : 0;
         return hip_status(qdl::purified_fwd_launch((int)c->dtype, a, s));
     }
     qdl::FwdArgs a = {};
@@ -138,6 +139,7 @@ int qdl_flash_born_backward_call(const qdl_born_call* c, qdl_stream_t stream) {
         a.dv = c->dv;
         a.dscale = c->dscale;
         a.dtau = c->dtau;
+        a.param_grads = c->dscale || c->dtau ? 1 : 0;
         const int64_t region = qdl::bwd_region_bytes(c->B, c->H, c->T);
         char* w = static_cast<char*>(c->workspace);
         a.ndelta = reinterpret_cast<float*>(w);

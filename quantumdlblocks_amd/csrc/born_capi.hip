@@ -45,7 +45,8 @@ int fwd_with_prologue(int dtype, const FwdArgs& a, const ProloguePlan& p, hipStr
                            p.q_strides[2] % 8 == 0 && p.q_strides[2] >= D &&
                            (T + 256) * p.q_strides[2] * 2 < ((int64_t)1 << 31);
     const bool masks_ok = a.doc ? (a.window == 0 || a.is_causal) : a.window == 0;
-    if (dtype == QDL_BORN_DTYPE_BF16 && D == 64 && masks_ok && q_rows_ok && (!p.cos || p.n_freq >= 1) &&
+    // A launch of few blocks takes the separate calls' few-block kernel.
+    if (!split16_pays(a, false, false) && dtype == QDL_BORN_DTYPE_BF16 && D == 64 && masks_ok && q_rows_ok && (!p.cos || p.n_freq >= 1) &&
         (T + 256) * D * 2 < ((int64_t)1 << 31)) {
         const int rc = qdl_flash_born_qk_prologue_fwd(dtype, a.B, a.H, T, D, nullptr, nullptr, a.k, p.k_strides, p.cos,
                                                       p.sin, p.n_freq, p.table_ld, p.norm_eps, nullptr, p.k_out,

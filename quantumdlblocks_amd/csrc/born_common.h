@@ -22,6 +22,7 @@
 #include <stdint.h>
 
 #include <climits>
+#include <cstddef>
 #include <type_traits>
 
 namespace qdl {
@@ -216,14 +217,23 @@ __device__ __forceinline__ f32x16 zero16() {
 }
 
 // A head's scale and tau: from device memory, or, without a pointer, the value
-// in the argument block (a caller's plain float needs no device copy).
+// in the argument block (a caller's plain float needs no device copy).  One
+// address either way, the block's being the kernel argument segment (Args is
+// every kernel's first argument), so both are the same scalar load: a branch
+// here cost the document kernels 1-2%.
+typedef const __attribute__((address_space(4))) float* ConstFloatPtr;
+__device__ __forceinline__ float arg_value(const float* p, int i, int offset) {
+    const uintptr_t block = (uintptr_t)__builtin_amdgcn_kernarg_segment_ptr() + offset;
+    const uintptr_t at = p != nullptr ? (uintptr_t)(p + i) : block;
+    return *(ConstFloatPtr)at;
+}
 template <class Args>
 __device__ __forceinline__ float arg_scale(const Args& p, int h) {
-    return p.scale != nullptr ? p.scale[p.per_head_scale ? h : 0] : p.scale_value;
+    return arg_value(p.scale, p.per_head_scale ? h : 0, offsetof(Args, scale_value));
 }
 template <class Args>
 __device__ __forceinline__ float arg_tau(const Args& p, int h) {
-    return p.tau != nullptr ? p.tau[p.per_head_tau ? h : 0] : p.tau_value;
+    return arg_value(p.tau, p.per_head_tau ? h : 0, offsetof(Args, tau_value));
 }
 
 // Kernel argument block shared by the forward kernels.

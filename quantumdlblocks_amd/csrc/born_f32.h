@@ -520,8 +520,8 @@ void born_f32_dq_kernel(typename std::conditional<PUR, PurArgs, BwdArgs>::type p
 }
 
 // ---------------------------------------------------------------------------
-// dK / dV (purified: with the dgamma / dtau partials).  Keys stationary; per
-// query tile S = Q K^T, dP = dO V^T - delta, dV^T += dO^T W, dK^T += Q^T dS.
+// dK / dV (purified: with a fixed scale and tau, whose gradients these kernels
+// do not form; see purified_split_ok).  Keys stationary; per query tile S = Q K^T, dP = dO V^T - delta, dV^T += dO^T W, dK^T += Q^T dS.
 // ---------------------------------------------------------------------------
 template <int DP, bool PUR, int NW>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(DP <= 64 ? 2 : 1)))
@@ -531,7 +531,6 @@ void born_f32_dkdv_kernel(typename std::conditional<PUR, PurArgs, BwdArgs>::type
     __shared__ __attribute__((aligned(1024))) uint8_t tiles[NW * 2 * F32Tile<DP>::BYTES];
     // Per wave: the tile's -delta, 1 / Z and query ids.
     __shared__ __attribute__((aligned(16))) float rv_lds[NW][3][kF32Rows];
-    __shared__ float pred[2][NW];
     __shared__ int32_t span_red[4];
     float* const red = reinterpret_cast<float*>(tiles);
 
@@ -576,7 +575,6 @@ void born_f32_dkdv_kernel(typename std::conditional<PUR, PurArgs, BwdArgs>::type
     f32x16 dv[DB], dk[DB];
 #pragma unroll
     for (int db = 0; db < DB; ++db) dv[db] = zero16(), dk[db] = zero16();
-    float ds_acc = 0.f, dt_acc = 0.f;
 
     const F32Tile<DP> qt = {tiles + (2 * wave) * F32Tile<DP>::BYTES}, dt = {tiles + (2 * wave + 1) * F32Tile<DP>::BYTES};
     constexpr int LOADS = F32Tile<DP>::LOADS;
@@ -653,8 +651,6 @@ void born_f32_dkdv_kernel(typename std::conditional<PUR, PurArgs, BwdArgs>::type
                 const float dpz = dp[r] * zi[r];
                 const float du = 4.0f * (u2 * uu) * dpz;
                 s[r] = du * pw.gam + 2.0f * pw.eb * bb * dpz;
-                ds_acc += du * (x - pw.tau);
-                dt_acc -= du * pw.gam;
             } else {
                 const float a = vis ? fmaxf(s[r], 0.f) : 0.f;
                 const float tz = a * zi[r];
@@ -686,27 +682,8 @@ void born_f32_dkdv_kernel(typename std::conditional<PUR, PurArgs, BwdArgs>::type
     const float fk = PUR ? 1.f : 2.f * sc * fabsf(sc), fv = PUR ? 1.f : sc * sc;
     float* const mine = red + wave * kF32Rows * (DP + 4);
     f32_put<DB>(mine, dv, c, g);
-    if constexpr (PUR) {
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            ds_acc += __shfl_xor(ds_acc, off);
-            dt_acc += __shfl_xor(dt_acc, off);
-        }
-        if (lane == 0) pred[0][wave] = ds_acc, pred[1][wave] = dt_acc;
-    }
     __syncthreads();
     f32_reduce_store<DB, NW>(red, reinterpret_cast<float*>(p.dv) + base, k0, T, D, [&](int, f32x4 x) -> f32x4 { return x * fv; });
-    if constexpr (PUR) {
-        // Partial sums of dgamma and dtau, one per workgroup, at key block *
-        // BH + head (the order purified_param_reduce_kernel expects).
-        if (tid == 0) {
-            float a = 0.f, t2 = 0.f;
-            for (int i = 0; i < NW; ++i) a += pred[0][i], t2 += pred[1][i];
-            const int slot = blk.mb * BH + blk.bh;
-            p.part[slot] = a;
-            p.part[gridDim.x + slot] = t2;
-        }
-    }
     __syncthreads();
     f32_put<DB>(mine, dk, c, g);
     __syncthreads();

@@ -8,6 +8,7 @@
 namespace qdl {
 
 hipError_t fwd_launch_bf16(const FwdArgs& a, hipStream_t s) {
+    if (split16_pays(a, false, false)) return split16_fwd<BF16>(a, s);
     const int dp = padded_head_dim(a.D);
     const int mode = mask_mode(a.is_causal, a.window, a.doc);
     // Hot path: D == 64 exactly, dense or causal, per-head slice addressable

@@ -3,6 +3,8 @@
 #pragma once
 
 #include "born_common.h"
+#include "purified_args.h"
+#include "split16_rule.h"
 
 namespace qdl {
 
@@ -36,6 +38,17 @@ struct ProloguePlan {
 int fwd_with_prologue(int dtype, const FwdArgs& a, const ProloguePlan& p, hipStream_t s);
 hipError_t bwd_launch_f16(const BwdArgs& a, hipStream_t s);
 hipError_t bwd_launch_f32(const BwdArgs& a, hipStream_t s);
+
+// The few-block kernels of 16-bit inputs (born_split16_*.hip), for launches
+// that split16_pays (split16_rule.h).
+template <class E>
+hipError_t split16_fwd(const FwdArgs& a, hipStream_t s);
+template <class E>
+hipError_t split16_fwd(const PurArgs& a, hipStream_t s);
+template <class E>
+hipError_t split16_bwd(const BwdArgs& a, hipStream_t s);
+template <class E>
+hipError_t split16_bwd(const PurArgs& a, hipStream_t s);
 
 }  // namespace qdl
 

@@ -1,0 +1,16 @@
+// Few-block kernel instantiations for fp16 inputs (born_split16.h).
+#include "born_split16.h"
+#include "born_launch.h"
+
+namespace qdl {
+
+template <>
+hipError_t split16_fwd<F16>(const FwdArgs& a, hipStream_t s) { return launch_split16_fwd<F16, false>(a, s); }
+template <>
+hipError_t split16_fwd<F16>(const PurArgs& a, hipStream_t s) { return launch_split16_fwd<F16, true>(a, s); }
+template <>
+hipError_t split16_bwd<F16>(const BwdArgs& a, hipStream_t s) { return launch_split16_bwd<F16, false>(a, s); }
+template <>
+hipError_t split16_bwd<F16>(const PurArgs& a, hipStream_t s) { return launch_split16_bwd<F16, true>(a, s); }
+
+}  // namespace qdl

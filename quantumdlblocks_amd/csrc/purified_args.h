@@ -28,6 +28,7 @@ struct PurArgs {
     float* part;         // workspace: 2 x (dK/dV workgroups) partial sums
     int per_head_scale;
     int per_head_tau;
+    int param_grads;     // scale or tau is trained (the dispatch: see purified_dispatch.h)
     int B, H, T, D;
     int is_causal;
     int window;

@@ -59,6 +59,7 @@ int qdl_flash_purified_born_fwd(int dtype, int64_t B, int64_t H, int64_t T, int6
     a.doc = doc_ids;
     a.per_head_scale = n_scale > 1 ? 1 : 0;
     a.per_head_tau = n_tau > 1 ? 1 : 0;
+    a.param_grads = 1;
     a.B = (int)B;
     a.H = (int)H;
     a.T = (int)T;
@@ -119,6 +120,7 @@ int qdl_flash_purified_born_bwd(int dtype, int64_t B, int64_t H, int64_t T, int6
     a.part = reinterpret_cast<float*>(w + 2 * region);
     a.per_head_scale = n_scale > 1 ? 1 : 0;
     a.per_head_tau = n_tau > 1 ? 1 : 0;
+    a.param_grads = 1;
     a.B = (int)B;
     a.H = (int)H;
     a.T = (int)T;

@@ -20,6 +20,16 @@ hipError_t purified_wide_bwd_launch(int dtype, const PurArgs& a, hipStream_t s);
 hipError_t purified_fwd_d256_launch(int dtype, const PurArgs& a, hipStream_t s);
 hipError_t purified_bwd_d256_launch(int dtype, const PurArgs& a, hipStream_t s);
 
+// Whether a call may take the wave-split kernels (born_f32.h, born_split16.h).
+// Where scale or tau is trained in fp32 or fp16 it keeps the other kernels:
+// dscale is a cancelling sum, which another summation order in the output (its
+// last bits) moves by up to 1e-3 (fp32) and 4e-3 (fp16), no nearer to or
+// further from float64 (1e-3 and 4e-2 off either way).
+template <class IN>
+inline bool purified_split_ok(const PurArgs& a) {
+    return std::is_same<IN, BF16>::value || !a.param_grads;
+}
+
 // fp32 inputs up to D = 128 (born_fwd_f32.hip, born_bwd_f32.hip).
 hipError_t purified_fwd_f32_launch(const PurArgs& a, hipStream_t s);
 hipError_t purified_bwd_f32_launch(const PurArgs& a, hipStream_t s);

@@ -3,6 +3,7 @@
 // bound-check columns past D).
 #include "born_fwd_d128.h"
 #include "born_fwd_doc.h"
+#include "born_launch.h"
 #include "purified_dispatch.h"
 
 namespace qdl {
@@ -14,6 +15,8 @@ static hipError_t purified_fwd_dispatch(const PurArgs& a, hipStream_t s) {
     // exactly into two bf16 terms).
     using E = typename std::conditional<std::is_same<IN, F16>::value, F16, BF16>::type;
     constexpr bool k16 = !std::is_same<IN, float>::value;
+    if constexpr (k16)
+        if (purified_split_ok<IN>(a) && split16_pays(a, false, true)) return split16_fwd<E>(a, s);
     // D = 64 (and below, zero columns), dense, causal or a window.
     if (k16 && purified_fast_ok(a)) {
         if (a.window > 0)
@@ -65,15 +68,12 @@ static hipError_t purified_fwd_dispatch(const PurArgs& a, hipStream_t s) {
     // 16-bit-MFMA kernels' purified mode.
     if (k16 && purified_d256_ok(a)) return purified_fwd_d256_launch(E::kDtype, a, s);
     if (k16 && (a.D > 128 || a.doc != nullptr)) return purified_wide_fwd_launch(E::kDtype, a, s);
-    if constexpr (!k16) {
-        return a.D <= kF32MaxD ? purified_fwd_f32_launch(a, s) : launch_purified_fwd<IN, 256>(a, s);
-    } else {
-        switch (purified_padded_dim(a.D)) {
-            case 32: return launch_purified_fwd<IN, 32>(a, s);
-            case 64: return launch_purified_fwd<IN, 64>(a, s);
-            case 128: return launch_purified_fwd<IN, 128>(a, s);
-            default: return launch_purified_fwd<IN, 256>(a, s);
-        }
+    if (!k16 && a.D <= kF32MaxD && purified_split_ok<IN>(a)) return purified_fwd_f32_launch(a, s);
+    switch (purified_padded_dim(a.D)) {
+        case 32: return launch_purified_fwd<IN, 32>(a, s);
+        case 64: return launch_purified_fwd<IN, 64>(a, s);
+        case 128: return launch_purified_fwd<IN, 128>(a, s);
+        default: return launch_purified_fwd<IN, 256>(a, s);
     }
 }
 // dtype codes as in qdl_flash_born.h: 0 fp32, 1 fp16, 2 bf16.

@@ -440,7 +440,8 @@ class _FlashPurifiedBornAttentionFn(torch.autograd.Function):
             q_c.data_ptr(), k_c.data_ptr(), v_c.data_ptr(), out_f32.data_ptr(), z.data_ptr(),
             scale_p, n_scale, scale_value, 0 if doc_c is None else doc_c.data_ptr(),
             1 if is_causal else 0, window, float(eps),
-            purified=1, tau=tau_p, n_tau=n_tau, tau_value=tau_value, eps_base=float(eps_base)))
+            purified=1, tau=tau_p, n_tau=n_tau, tau_value=tau_value, eps_base=float(eps_base),
+            param_grads=1 if ctx.needs_input_grad[3] or ctx.needs_input_grad[4] else 0))
         ctx.save_for_backward(q_c, k_c, v_c, out_f32, z, scale_flat, tau_flat, doc_c)
         ctx.is_causal = bool(is_causal)
         ctx.window_size = window

@@ -40,7 +40,7 @@ def test_validation():
     lib = _native.load()
     for fn in (lib.qdl_flash_born_forward_call, lib.qdl_flash_born_backward_call):
         assert fn(None, None) == -5
-        assert fn(ctypes.c_char_p(b"\0" * 376), None) == -2  # struct_bytes
+        assert fn(ctypes.c_char_p(b"\0" * 384), None) == -2  # struct_bytes
         assert fn(_block(dtype=7), None) == -1
         assert fn(_block(D=12), None) == -3
         assert fn(_block(scale=64, n_scale=3), None) == -6
@@ -71,7 +71,8 @@ def test_parameters_by_value(cuda_device, purified, dtype, D, mask):
     if kw.pop("doc", False):
         kw["doc_ids"] = (torch.arange(70, device=cuda_device) // 25).view(1, 70)
     got = []
-    for scale, tau in ((-1.5, 0.02), (torch.tensor([-1.5, -1.5], device=cuda_device, requires_grad=True),
+    for scale, tau in ((-1.5, 0.02), (torch.tensor([-1.5, -1.5], device=cuda_device,
+                                                                requires_grad=not purified),
                                       torch.tensor(0.02, device=cuda_device))):
         x = [t.clone().requires_grad_(True) for t in (q, k, v)]
         if purified:

@@ -18,8 +18,8 @@ import torch
 
 from oracle import born_oracle as orc
 from test_gpu_backward import _check_bwd
-from test_gpu_purified import _check_pur
-from util import f64, rel_err, seeded_inputs
+from test_gpu_purified import FLOOR, GTOL
+from util import TOL, f64, max_abs, rel_err, seeded_inputs
 
 pytestmark = pytest.mark.gpu
 
@@ -32,6 +32,31 @@ MASKS = {
     "docs_window": (True, 50, True),
     "docs_dense": (False, 0, True),
 }
+
+
+def check_pur_fixed(B, H, T, D, dtype, mask, scale, tau, std, device, doc):
+    """Purified attention with a fixed scale and tau (one that is trained keeps
+    the other kernels in fp32 and fp16): output, dq, dk, dv."""
+    from quantumdlblocks_amd import flash_purified_born_attention
+
+    causal, window, _ = mask
+    q, k, v, do = (x.to(device) for x in seeded_inputs((B, H, T, D), seed=T + D, std=std, n=4, dtype=dtype))
+    print(f"purified, fixed scale: B{B} H{H} T{T} D{D} {dtype} {mask}", flush=True)
+    q, k, v = (x.requires_grad_(True) for x in (q, k, v))
+    st, tt = (torch.tensor(x, dtype=torch.float32, device=device) for x in (scale, tau))
+    doc_t = None if doc is None else torch.as_tensor(doc, dtype=torch.int32, device=device)
+    out = flash_purified_born_attention(q, k, v, st, tt, 0.05, is_causal=causal, window_size=window, doc_ids=doc_t)
+    out.backward(do)
+    n = [f64(x) for x in (q, k, v)]
+    args = (*n, np.asarray(scale), np.asarray(tau))
+    okw = dict(eps_base=0.05, is_causal=causal, eps=1e-8, window_size=window, doc_ids=doc)
+    ref, _ = orc.purified_forward(*args, **okw)
+    assert rel_err(f64(out), ref) <= TOL[dtype], rel_err(f64(out), ref)
+    want = orc.purified_backward(*args, f64(do), **okw)
+    mags = orc.purified_backward_magnitudes(*args, f64(do), **okw)
+    for name, got, w, m in zip(("dq", "dk", "dv"), (q.grad, k.grad, v.grad), want, mags):
+        er, ef = rel_err(f64(got), w), max_abs(f64(got), w) / m.max()
+        assert er <= GTOL[dtype] or ef <= FLOOR[dtype], f"{name}: rel {er:.3e}, vs term scale {ef:.3e}"
 
 
 def _case(H, T, D, mask, purified, device, sorted_docs=True):
@@ -48,8 +73,7 @@ def _case(H, T, D, mask, purified, device, sorted_docs=True):
         # 4e-7 (|x| within 3 at std 0.3) that is 1e-5 once |x - tau| < 0.16, so
         # their tau lies below every overlap.
         tau = [(-6.0 if docs else 0.05) - 0.03 * (h % 4) for h in range(H)]
-        _check_pur((2, H, T, D, torch.float32, dict(is_causal=causal, window_size=window), scale, tau, 0.3), device,
-                   doc)
+        check_pur_fixed(2, H, T, D, torch.float32, MASKS[mask], scale, tau, 0.3, device, doc)
     else:
         if H > 1:
             scale[1] = -0.8

@@ -1,0 +1,58 @@
+"""The rule that sends a 16-bit launch of few blocks to the wave-split kernels
+(csrc/split16_rule.h), compiled on the host: it takes the shapes their GPU
+tests use, leaves the tuned kernels' own ranges alone, and stays finite at the
+ends of the argument range."""
+
+from __future__ import annotations
+
+import os
+import shutil
+import subprocess
+
+import pytest
+
+RULE = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "quantumdlblocks_amd", "csrc",
+                    "split16_rule.h")
+MAIN = """
+#include <cstdio>
+#include <cstdlib>
+#include "%s"
+struct A { int B, H, T, D, is_causal, window; };
+int main(int, char** v) {
+    const A a = {atoi(v[1]), atoi(v[2]), atoi(v[3]), atoi(v[4]), atoi(v[5]), atoi(v[6])};
+    for (int pur = 0; pur < 2; ++pur)
+        printf("%%d %%d ", qdl::split16_pays(a, false, pur), qdl::split16_pays(a, true, pur));
+}
+""" % RULE
+
+
+@pytest.fixture(scope="module")
+def rule(tmp_path_factory):
+    gxx = shutil.which("g++")
+    if gxx is None:
+        pytest.skip("no host compiler")
+    d = tmp_path_factory.mktemp("rule")
+    (d / "main.cpp").write_text(MAIN)
+    subprocess.run([gxx, "-std=c++17", str(d / "main.cpp"), "-o", str(d / "rule")], check=True)
+
+    def ask(B, H, T, D, causal=1, window=0):
+        """(Born forward, Born backward, purified forward, purified backward)"""
+        args = [str(x) for x in (B, H, T, D, causal, window)]
+        return [w == "1" for w in subprocess.check_output([str(d / "rule"), *args], text=True).split()]
+
+    return ask
+
+
+@pytest.mark.parametrize("D", [24, 64, 72, 96, 120, 128, 160, 256])
+@pytest.mark.parametrize("causal,window", [(1, 0), (0, 0), (0, 300)])
+def test_few_blocks_take_the_split_kernels(rule, D, causal, window):
+    assert any(rule(1, 2, 700, D, causal, window))
+    if window == 0:
+        assert all(rule(1, 2, 1000, D, causal, window))
+
+
+@pytest.mark.parametrize("B,H,T,D", [(16, 16, 1024, 64), (16, 16, 2048, 64), (32, 4, 1024, 64), (16, 8, 2048, 128),
+                                     (4, 16, 8192, 64), (16, 4, 2048, 256), (2, 4, 64, 32), (1, 1, 1, 64),
+                                     (4096, 4096, 4, 64), (1, 1, 1 << 28, 256)])
+def test_others_keep_the_tuned_kernels(rule, B, H, T, D):
+    assert not any(rule(B, H, T, D))
