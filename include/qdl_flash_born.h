@@ -189,7 +189,8 @@ int qdl_flash_purified_born_bwd(int dtype, int64_t B, int64_t H, int64_t T,
  *     plain number needs no device copy and no synchronisation;
  *   - dscale / dtau == NULL: that gradient is not wanted, and the launches
  *     that reduce it are left out;
- *   - purified != 0 selects the purified weights (out is then fp32), prologue
+ *   - purified != 0 selects the purified weights (out is then fp32; out16 takes
+ *     the output rounded to the element type), prologue
  *     != 0 the fused Q/K prologue (Born forward).
  * param_grads keeps fp32 and fp16 purified calls whose scale or tau is trained
  * on the kernels of the positional entry points: dscale is a cancelling sum,
@@ -215,6 +216,7 @@ typedef struct qdl_born_call {
     int64_t n_tau;
     double tau_value;
     double eps_base;
+    void *out16;         /* purified forward, 16-bit: the output in the element type (out may then be NULL: no backward) */
     int64_t param_grads; /* purified forward: != 0 if the backward will be asked for dscale or dtau */
     /* backward */
     const void *dout;

@@ -51,18 +51,18 @@ class NativeLibraryError(RuntimeError):
 
 # qdl_born_call: every field 8 bytes ("q" integers and addresses, "d" doubles).
 # The forward leaves the backward's fields zero.
-_CALL = struct.Struct("@" + "q" * 6 + "q" * 5 + "qqd" + "qqqd" + "qqqddq" + "q" * 8 + "q" + "q" * 6 + "qqqqd" + "q" * 4)
+_CALL = struct.Struct("@" + "q" * 6 + "q" * 5 + "qqd" + "qqqd" + "qqqddqq" + "q" * 8 + "q" + "q" * 6 + "qqqqd" + "q" * 4)
 _NO_PROLOGUE = (0,) * 7 + (0, 0, 0, 0, 0.0) + (0,) * 4
 
 
 def pack_call(dtype, B, H, T, D, q, k, v, out, z, scale, n_scale, scale_value, doc, causal, window, eps,
-              purified=0, tau=0, n_tau=0, tau_value=0.0, eps_base=0.0, param_grads=0,
+              purified=0, tau=0, n_tau=0, tau_value=0.0, eps_base=0.0, out16=0, param_grads=0,
               dout=0, dq=0, dk=0, dv=0, dscale=0, dtau=0, workspace=0, workspace_bytes=0,
               prologue=_NO_PROLOGUE) -> bytes:
     """The argument block of qdl_flash_born_forward_call / _backward_call;
     ``prologue``: the fields from ``prologue`` on."""
     return _CALL.pack(_CALL.size, dtype, B, H, T, D, q, k, v, out, z, scale, n_scale, scale_value, doc, causal, window,
-                      eps, purified, tau, n_tau, tau_value, eps_base, param_grads, dout, dq, dk, dv, dscale, dtau, workspace,
+                      eps, purified, tau, n_tau, tau_value, eps_base, out16, param_grads, dout, dq, dk, dv, dscale, dtau, workspace,
                       workspace_bytes, *prologue)
 
 

@@ -73,7 +73,11 @@ int qdl_flash_born_forward_call(const qdl_born_call* c, qdl_stream_t stream) {
     int rc = check(c);
     if (rc != QDL_BORN_OK) return rc;
     if (c->B * c->H * c->T == 0) return QDL_BORN_OK;
-    if (!c->q || !c->k || !c->v || !c->out || !c->z) return QDL_BORN_E_NULL;
+    // The purified output in the element type: 16-bit inputs.
+    const bool has16 = c->purified && c->out16;
+    if (has16 && c->dtype == QDL_BORN_DTYPE_F32) return QDL_BORN_E_DTYPE;
+    if (!c->q || !c->k || !c->v || (!c->out && !has16) || !c->z) return QDL_BORN_E_NULL;
+    if (has16 && !aligned16(c->out16)) return QDL_BORN_E_ALIGN;
     if (c->prologue) {
         if (c->cos_table && (!c->sin_table || c->n_freq < 0 || c->n_freq > c->D / 2 || c->table_ld < c->n_freq))
             return QDL_BORN_E_TABLE;
@@ -89,6 +93,7 @@ int qdl_flash_born_forward_call(const qdl_born_call* c, qdl_stream_t stream) {
         qdl::PurArgs a = {};
         fill_purified(a, c);
         a.o = static_cast<float*>(c->out);
+        a.o16 = c->out16;
         a.z = c->z;
         a.param_grads = c->param_grads ? 1 : 0;
         return hip_status(qdl::purified_fwd_launch((int)c->dtype, a, s));

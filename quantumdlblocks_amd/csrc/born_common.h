@@ -294,6 +294,33 @@ struct BwdArgs {
     float eps;
 };
 
+// The purified forward's outputs.  Read again from the kernel argument segment
+// where they are stored: held through the tile loop they cost scalar registers
+// that it has none to spare of.
+struct PurOut {
+    float* o;
+    uint16_t* o16;
+};
+template <class Args>
+__device__ __forceinline__ PurOut pur_out() {
+    typedef const __attribute__((address_space(4))) Args* ArgPtr;
+    ArgPtr a = (ArgPtr)(uintptr_t)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(a));
+    const PurOut r = {a->o, reinterpret_cast<uint16_t*>(a->o16)};
+    return r;
+}
+// Four consecutive values: fp32 for the backward, and rounded to the input
+// dtype for the caller (a separate pass over the fp32 output read it again
+// whole: 29 us of B4 H16 T8192 D64's 720 us step).
+template <class E>
+__device__ __forceinline__ void pur_store4(const PurOut& out, size_t at, f32x4 w) {
+    if (out.o != nullptr) *reinterpret_cast<f32x4*>(out.o + at) = w;
+    if (out.o16 != nullptr) {
+        const u32x2 x = {E::pack(w[0], w[1]), E::pack(w[2], w[3])};
+        *reinterpret_cast<u32x2*>(out.o16 + at) = x;
+    }
+}
+
 // Fixed number of partial sums per dscale output (deterministic reduction).
 constexpr int DSCALE_CHUNKS = 128;
 

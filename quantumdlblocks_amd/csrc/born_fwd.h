@@ -431,7 +431,7 @@ void born_fwd16_kernel(typename std::conditional<PUR, PurArgs, FwdArgs>::type p)
     float* __restrict__ Zp = p.z + (size_t)bh * T;
     if constexpr (PUR) {
         // O = acc / (Z + eps) and Z + eps in fp32.
-        float* __restrict__ O32 = p.o + base;
+        const PurOut dst = pur_out<PurArgs>();
 #pragma unroll
         for (int qb = 0; qb < NQB; ++qb) {
             const float zl = zacc[qb][0] + zacc[qb][1];
@@ -446,7 +446,7 @@ void born_fwd16_kernel(typename std::conditional<PUR, PurArgs, FwdArgs>::type p)
                         if (d < D) {
                             const f32x16& o = oacc[db][qb];
                             const f32x4 w = {o[4 * j] / zd, o[4 * j + 1] / zd, o[4 * j + 2] / zd, o[4 * j + 3] / zd};
-                            *reinterpret_cast<f32x4*>(O32 + (size_t)qi * D + d) = w;
+                            pur_store4<E>(dst, base + (size_t)qi * D + d, w);
                         }
                     }
                 }

@@ -423,7 +423,6 @@ void born_fwd16_d128_kernel(typename std::conditional<PUR, PurArgs, FwdArgs>::ty
     };
 
     uint16_t* __restrict__ O = reinterpret_cast<uint16_t*>(p.o) + base;
-    float* __restrict__ O32 = reinterpret_cast<float*>(p.o) + base;  // purified: fp32 rows
     float* __restrict__ Zp = p.z + (size_t)bh * T;
     const float s2 = (sq_pre > 0.f) ? (sc / sq_pre) * (sc / sq_pre) : 0.f;
     const float eps_s = (p.eps == 0.f) ? 0.f : p.eps / s2;
@@ -487,6 +486,7 @@ void born_fwd16_d128_kernel(typename std::conditional<PUR, PurArgs, FwdArgs>::ty
     // merges a row's pieces into whole lines before they reach HBM
     // (non-temporal stores wrote them partial, 2.3x the output bytes).
     auto store_pur = [&](int mb) __attribute__((always_inline)) {
+        const PurOut dst = pur_out<PurArgs>();
         const float zl = zacc[0] + zacc[1];
         const float zd = zl + __shfl_xor(zl, 32) + p.eps;
         const int qi = mb * BM + 32 * wave + c;
@@ -499,7 +499,7 @@ void born_fwd16_d128_kernel(typename std::conditional<PUR, PurArgs, FwdArgs>::ty
                     const f32x4 w = {o[4 * j] / zd, o[4 * j + 1] / zd, o[4 * j + 2] / zd, o[4 * j + 3] / zd};
                     const int col = db * 32 + 8 * j + 4 * g;
                     if (!PAD || col < D)
-                        *reinterpret_cast<f32x4*>(O32 + (size_t)qi * D + col) = w;
+                        pur_store4<E>(dst, base + (size_t)qi * D + col, w);
                 }
             if (g == 0) __builtin_nontemporal_store(zd, Zp + qi);
         }

@@ -400,7 +400,7 @@ void born_fwd16_d256_kernel(typename std::conditional<PUR, PurArgs, FwdArgs>::ty
         const float zl = zacc[0] + zacc[1];
         const float zd = zl + __shfl_xor(zl, 32) + p.eps;
         if (qrow < T) {
-            float* __restrict__ O32 = p.o + base;
+            const PurOut dst = pur_out<PurArgs>();
 #pragma unroll
             for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -408,7 +408,7 @@ void born_fwd16_d256_kernel(typename std::conditional<PUR, PurArgs, FwdArgs>::ty
                     const f32x4 w = {oacc[db][4 * j] / zd, oacc[db][4 * j + 1] / zd, oacc[db][4 * j + 2] / zd,
                                      oacc[db][4 * j + 3] / zd};
                     const int col = db * 32 + 8 * j + 4 * g;
-                    if (!PAD || col < D) *reinterpret_cast<f32x4*>(O32 + (size_t)qrow * D + col) = w;
+                    if (!PAD || col < D) pur_store4<E>(dst, base + (size_t)qrow * D + col, w);
                 }
             if (g == 0) __builtin_nontemporal_store(zd, p.z + (size_t)bh * T + qrow);
         }

@@ -595,7 +595,7 @@ void born_fwd16_doc_kernel(
     float* __restrict__ Zp = p.z + (size_t)bh * T;
     if constexpr (PUR) {
         // Purified: O = acc / (Z + eps) in fp32, stored from the accumulators.
-        float* __restrict__ O32 = p.o + base;
+        const PurOut dst = pur_out<PurArgs>();
 #pragma unroll
         for (int qb = 0; qb < NQB; ++qb) {
             const float zl = zacc[qb][0] + zacc[qb][1];
@@ -609,7 +609,7 @@ void born_fwd16_doc_kernel(
                         const f32x16& o = oacc[db][qb];
                         const f32x4 w = {o[4 * j] / zd, o[4 * j + 1] / zd, o[4 * j + 2] / zd, o[4 * j + 3] / zd};
                         // plain store: L2 merges each row's 32-byte pieces into whole lines
-                        *reinterpret_cast<f32x4*>(O32 + (size_t)qi * DP + db * 32 + 8 * j + 4 * g) = w;
+                        pur_store4<E>(dst, base + (size_t)qi * DP + db * 32 + 8 * j + 4 * g, w);
                     }
                 if (g == 0) __builtin_nontemporal_store(zd, Zp + qi);
             }

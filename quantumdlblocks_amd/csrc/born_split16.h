@@ -135,7 +135,7 @@ __device__ __forceinline__ void split_put(float* red, const f32x16 (&acc)[DB], i
 }
 
 // The waves' shares summed in wave order and finished by finish(row, sum), to
-// rows r0 .. of a (T, D) slice: 16-bit (out) or fp32 (out32).
+// rows r0 .. of a (T, D) slice: 16-bit (out) and fp32 (out32), or one of them.
 template <class E, int DB, class F>
 __device__ __forceinline__ void split_store(const float* red, uint16_t* out, float* out32, int r0, int T, int D,
                                             F&& finish) {
@@ -393,8 +393,8 @@ void born_split16_fwd_kernel(typename std::conditional<PUR, PurArgs, FwdArgs>::t
         uint16_t* out;
         float* out32 = nullptr;
         if constexpr (PUR) {
-            out = nullptr;
-            out32 = p.o + base;
+            out = p.o16 != nullptr ? reinterpret_cast<uint16_t*>(p.o16) + base : nullptr;
+            out32 = p.o != nullptr ? p.o + base : nullptr;
         } else {
             out = reinterpret_cast<uint16_t*>(p.o) + base;
         }

@@ -265,7 +265,6 @@ void purified_fwd_kernel(PurArgs p) {
 
     const float zd = zacc + __shfl_xor(zacc, 32) + p.eps;
     if (qi < T) {
-        float* __restrict__ O = p.o + base;
 #pragma unroll
         for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -274,7 +273,10 @@ void purified_fwd_kernel(PurArgs p) {
                 if (d < D) {
                     const f32x4 w = {oacc[db][4 * j] / zd, oacc[db][4 * j + 1] / zd, oacc[db][4 * j + 2] / zd,
                                      oacc[db][4 * j + 3] / zd};
-                    *reinterpret_cast<f32x4*>(O + (size_t)qi * D + d) = w;
+                    const size_t at = base + (size_t)qi * D + d;
+                    if (p.o != nullptr) *reinterpret_cast<f32x4*>(p.o + at) = w;
+                    if constexpr (!std::is_same<IN, float>::value)
+                        if (p.o16 != nullptr) PurIO<IN>::store4(p.o16, at, w);
                 }
             }
         if (g == 0) p.z[(size_t)bh * T + qi] = zd;

@@ -9,7 +9,8 @@ struct PurArgs {
     const void* q;
     const void* k;
     const void* v;
-    float* o;            // forward: (B, H, T, D) fp32 output
+    float* o;            // forward: (B, H, T, D) fp32 output, or nullptr: o16 alone
+    void* o16;           // forward, 16-bit inputs: the output in the input dtype too, or nullptr
     float* z;            // forward: (B, H, T) fp32, Z = sum p + eps
     const float* o_in;   // backward: the forward's fp32 output
     const void* dout;    // backward: upstream gradient, input dtype

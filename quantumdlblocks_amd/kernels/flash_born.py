@@ -432,15 +432,20 @@ class _FlashPurifiedBornAttentionFn(torch.autograd.Function):
         dp = (D + 7) // 8 * 8
         q_c, k_c, v_c = _cast(q, target, dp), _cast(k, target, dp), _cast(v, target, dp)
         doc_c = None if doc_ids is None else _aligned(doc_ids.to(device=dev, dtype=torch.int32))
-        out_f32 = torch.empty((B, H, T, dp), dtype=torch.float32, device=dev)
+        # 16-bit: the kernel writes the output in the compute dtype too, and the
+        # fp32 one only for a backward.
+        out = torch.empty((B, H, T, dp), dtype=target, device=dev) if target != torch.float32 else None
+        out_f32 = None
+        if out is None or any(ctx.needs_input_grad[:5]):
+            out_f32 = torch.empty((B, H, T, dp), dtype=torch.float32, device=dev)
         z = torch.empty((B, H, T), dtype=torch.float32, device=dev)
         window = max(int(window_size), 0)
         _run_call(lib.qdl_flash_born_forward_call, "qdl_flash_born_forward_call (purified)", dev, _native.pack_call(
             _DTYPE_CODE[target], B, H, T, dp,
-            q_c.data_ptr(), k_c.data_ptr(), v_c.data_ptr(), out_f32.data_ptr(), z.data_ptr(),
+            q_c.data_ptr(), k_c.data_ptr(), v_c.data_ptr(), 0 if out_f32 is None else out_f32.data_ptr(), z.data_ptr(),
             scale_p, n_scale, scale_value, 0 if doc_c is None else doc_c.data_ptr(),
             1 if is_causal else 0, window, float(eps),
-            purified=1, tau=tau_p, n_tau=n_tau, tau_value=tau_value, eps_base=float(eps_base),
+            out16=0 if out is None else out.data_ptr(), purified=1, tau=tau_p, n_tau=n_tau, tau_value=tau_value, eps_base=float(eps_base),
             param_grads=1 if ctx.needs_input_grad[3] or ctx.needs_input_grad[4] else 0))
         ctx.save_for_backward(q_c, k_c, v_c, out_f32, z, scale_flat, tau_flat, doc_c)
         ctx.is_causal = bool(is_causal)
@@ -450,8 +455,9 @@ class _FlashPurifiedBornAttentionFn(torch.autograd.Function):
         ctx.values = (scale_value, tau_value)
         ctx.shapes = tuple((p.shape, p.dtype) if isinstance(p, torch.Tensor) else None for p in (scale, tau))
         ctx.dtypes = (q.dtype, k.dtype, v.dtype)
-        out = out_f32 if dp == D else out_f32[..., :D]
-        return out.to(target)
+        if out is None:
+            out = out_f32
+        return out if dp == D else out[..., :D].contiguous()
 
     @staticmethod
     def backward(ctx, do: torch.Tensor):

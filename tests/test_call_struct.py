@@ -40,7 +40,7 @@ def test_validation():
     lib = _native.load()
     for fn in (lib.qdl_flash_born_forward_call, lib.qdl_flash_born_backward_call):
         assert fn(None, None) == -5
-        assert fn(ctypes.c_char_p(b"\0" * 384), None) == -2  # struct_bytes
+        assert fn(ctypes.c_char_p(b"\0" * 392), None) == -2  # struct_bytes
         assert fn(_block(dtype=7), None) == -1
         assert fn(_block(D=12), None) == -3
         assert fn(_block(scale=64, n_scale=3), None) == -6
@@ -113,3 +113,30 @@ def test_a_call_captures_with_a_plain_scale(cuda_device):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, flash_born_attention(q, k, v, 2.0))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32], ids=str)
+@pytest.mark.parametrize("D", [24, 40, 64, 96, 128, 200])
+@pytest.mark.parametrize("T", [60, 600])
+@pytest.mark.parametrize("mask", [dict(), dict(is_causal=False), dict(window_size=30), dict(doc=True),
+                                  dict(is_causal=False, window_size=20, doc=True)], ids=str)
+def test_purified_output_in_the_compute_dtype(cuda_device, dtype, D, T, mask):
+    """The kernels round the output to the compute dtype themselves: it is the
+    fp32 output (what a backward keeps) rounded to nearest, and a call without
+    a backward, which writes no fp32 output, returns the same."""
+    from quantumdlblocks_amd import flash_purified_born_attention
+
+    g = torch.Generator("cpu").manual_seed(D)
+    q, k, v = (torch.randn(1, 2, T, D, generator=g).mul(0.3).to(cuda_device, dtype) for _ in range(3))
+    kw = dict(mask)
+    if kw.pop("doc", False):
+        kw["doc_ids"] = (torch.arange(T, device=cuda_device) // 25).view(1, T)
+    with torch.no_grad():
+        plain = flash_purified_born_attention(q, k, v, **kw)
+    out = flash_purified_born_attention(q.requires_grad_(True), k, v, **kw)
+    kept = out.grad_fn.saved_tensors[3]  # the fp32 output
+    assert kept.dtype == torch.float32
+    assert plain.dtype == out.dtype == dtype and out.is_contiguous()
+    assert torch.equal(plain, out)
+    assert torch.equal(out, kept.to(dtype)[..., :D])
