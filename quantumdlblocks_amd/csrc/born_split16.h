@@ -25,6 +25,7 @@
 #include "born_f32.h"
 #include "born_fwd_fast.h"
 #include "purified_args.h"
+#include "split16_rule.h"
 
 namespace qdl {
 
@@ -48,17 +49,18 @@ struct Tile16 {
     }
     // Lane's byte offsets of a tile's loads within a (T, D) slice; chunks past
     // D read out of range (zeros).
-    __device__ __forceinline__ static void offsets(int (&off)[LOADS], int D, int lane) {
+    __device__ __forceinline__ static void offsets(uint32_t (&off)[LOADS], int D, int lane) {
 #pragma unroll
         for (int i = 0; i < LOADS; ++i) {
             const int slot = 64 * i + lane, row = slot / CPR, chunk = (slot % CPR) ^ swz(row);
-            off[i] = 8 * chunk < D ? row * D * 2 + 16 * chunk : kBufOOB;
+            off[i] = 8 * chunk < D ? (uint32_t)(row * D * 2 + 16 * chunk) : kSplitPastD;
         }
     }
     // The rows from byte `at` of the slice (rows past T: out of range).
-    __device__ __forceinline__ void issue(i32x4 slice, const int (&off)[LOADS], int at) const {
+    __device__ __forceinline__ void issue(i32x4 slice, const uint32_t (&off)[LOADS], int at) const {
 #pragma unroll
-        for (int i = 0; i < LOADS; ++i) dma_load16(slice, lds_addr(lds + 1024 * i), off[i] + at);
+        for (int i = 0; i < LOADS; ++i)
+            dma_load16(slice, lds_addr(lds + 1024 * i), (int)split16_load_at(off[i], (uint32_t)at));
     }
     // A operand of a contraction over the head dim: row c, columns 16 ks + 8 g .. + 7.
     __device__ __forceinline__ u32x4 row(int ks, int c, int g) const {
@@ -254,7 +256,7 @@ void born_split16_fwd_kernel(typename std::conditional<PUR, PurArgs, FwdArgs>::t
     uint8_t* const ring = smem + wave * C::RING;
     auto kt = [&](int st) { return Tile{ring + st * 2 * Tile::BYTES}; };
     auto vt = [&](int st) { return Tile{ring + st * 2 * Tile::BYTES + Tile::BYTES}; };
-    int off[Tile::LOADS];
+    uint32_t off[Tile::LOADS];
     Tile::offsets(off, D, lane);
     const i32x4 rk = split_slice(K, T, D), rv = split_slice(V, T, D);
     // This wave's tile i; past the last one its loads are out of range and land
@@ -459,7 +461,7 @@ void born_split16_dq_kernel(typename std::conditional<PUR, PurArgs, BwdArgs>::ty
     uint8_t* const ring = smem + wave * C::RING;
     auto kt = [&](int st) { return Tile{ring + st * 2 * Tile::BYTES}; };
     auto vt = [&](int st) { return Tile{ring + st * 2 * Tile::BYTES + Tile::BYTES}; };
-    int off[Tile::LOADS];
+    uint32_t off[Tile::LOADS];
     Tile::offsets(off, D, lane);
     const i32x4 rk = split_slice(K, T, D), rv = split_slice(V, T, D);
     auto row0 = [&](int i) { return i < n ? 32 * (t_lo + wave + NW * i) : T; };
@@ -677,7 +679,7 @@ void born_split16_dkdv_kernel(typename std::conditional<PUR, PurArgs, BwdArgs>::
     uint8_t* const ring = smem + wave * C::RING;
     auto dt = [&](int st) { return Tile{ring + st * 2 * Tile::BYTES}; };
     auto qt = [&](int st) { return Tile{ring + st * 2 * Tile::BYTES + Tile::BYTES}; };
-    int off[Tile::LOADS];
+    uint32_t off[Tile::LOADS];
     Tile::offsets(off, D, lane);
     const i32x4 rq = split_slice(Q, T, D), rd = split_slice(dO, T, D);
     const i32x4 rnd = split_slice32(NDl, T), rzi = split_slice32(ZIl, T);

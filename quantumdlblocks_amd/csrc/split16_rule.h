@@ -77,12 +77,21 @@ inline void split16_times(int kernel, bool pur, int64_t bh, int64_t T, int D, bo
     *split = c.sa * (1.0 + 0.7 * (rounds - 1)) + (c.sc * chain > moved ? c.sc * chain : moved);
 }
 
+// The kernels address a (T, D) slice with 32-bit byte offsets, rows up to T + 256.
+constexpr bool split16_addressable(int64_t T) { return (T + 256) * 512 < ((int64_t)1 << 31); }
+
+// Byte offset of a load within a slice: a chunk's offset in its tile (kSplitPastD
+// for the chunks past D) and the tile's.  Unsigned, because the sum passes 2^31
+// for chunks past D: it stays past the slice's end and below 2^32 for every
+// addressable T (a signed sum overflows).
+constexpr uint32_t kSplitPastD = 0x7ffffff0u;
+constexpr uint32_t split16_load_at(uint32_t chunk, uint32_t tile) { return chunk + tile; }
+
 // bwd: dQ and dK/dV together (one side's row sums feed the other's kernel).
 template <class Args>
 inline bool split16_pays(const Args& a, bool bwd, bool pur) {
     const int64_t bh = (int64_t)a.B * a.H;
-    // The kernels address a (T, D) slice with 32-bit byte offsets.
-    if (((int64_t)a.T + 256) * 512 >= ((int64_t)1 << 31)) return false;
+    if (!split16_addressable(a.T)) return false;
     double tuned = 0, split = 0;
     for (int k = bwd ? kSplitDq : kSplitFwd; k <= (bwd ? kSplitDkdv : kSplitFwd); ++k) {
         double t, s;

@@ -56,3 +56,33 @@ def test_few_blocks_take_the_split_kernels(rule, D, causal, window):
                                      (4096, 4096, 4, 64), (1, 1, 1 << 28, 256)])
 def test_others_keep_the_tuned_kernels(rule, B, H, T, D):
     assert not any(rule(B, H, T, D))
+
+
+OFFSETS = """
+#include <initializer_list>
+#include "%s"
+using namespace qdl;
+// In a constant expression an overflow of a signed sum is a compile error.
+constexpr int64_t kMaxT = (((int64_t)1 << 31) - 1) / 512 - 256;
+static_assert(split16_addressable(kMaxT) && !split16_addressable(kMaxT + 1), "the largest T");
+constexpr bool past_the_slice(int64_t T) {
+    for (int64_t D = 8; D <= 256; D += 8)
+        for (int64_t row : {(int64_t)0, T / 2, T}) {  // a tile's first row; T: a tile that is not there
+            const auto at = split16_load_at(kSplitPastD, (decltype(split16_load_at(0, 0)))(row * D * 2));
+            if ((int64_t)(uint32_t)at < T * D * 2 || (int64_t)(uint32_t)at + 16 > ((int64_t)1 << 32)) return false;
+        }
+    return true;
+}
+static_assert(past_the_slice(1) && past_the_slice(32) && past_the_slice(1000) && past_the_slice(kMaxT), "chunks past D");
+int main() {}
+""" % RULE
+
+
+def test_offsets_of_chunks_past_the_head_dim(tmp_path):
+    """Loads of the columns past D stay out of a slice's range, without
+    overflow, for every T that the kernels take."""
+    gxx = shutil.which("g++")
+    if gxx is None:
+        pytest.skip("no host compiler")
+    (tmp_path / "offsets.cpp").write_text(OFFSETS)
+    subprocess.run([gxx, "-std=c++17", "-fsyntax-only", str(tmp_path / "offsets.cpp")], check=True)
