@@ -43,6 +43,7 @@
 #include "born_common.h"
 #include "born_fwd_fast.h"
 #include "purified_args.h"
+#include "split16_rule.h"
 
 namespace qdl {
 
@@ -125,14 +126,11 @@ __device__ __forceinline__ void f32_issue_values(const void* v, int r0, int T, v
     if (lane < 8) dma_load16(rs, lds_addr(lds), 16 * lane);
 }
 
-// Block of a workgroup: the longest tile ranges first.  Where the whole launch
-// is resident at once, two workgroups per CU (257 to 512 of them), the second
-// half goes out shortest first, so that a CU pairs a long block with a short
-// one (B2 H8 T1000 D64 step: 159 -> 142 us).
+// Block of a workgroup: the longest tile ranges first (split_rank).
 struct SplitBlock {
     int bh, mb;
-    __device__ __forceinline__ SplitBlock(int bid, int grid, int BH, int nmb, bool longest_last) {
-        const int rank = grid <= 512 && bid >= 256 ? grid - 1 - (bid - 256) : bid;
+    __device__ __forceinline__ SplitBlock(int bid, int grid, int BH, int nmb, bool longest_last, bool two_per_cu) {
+        const int rank = split_rank(bid, grid, two_per_cu);
         bh = rank % BH;
         mb = longest_last ? nmb - 1 - rank / BH : rank / BH;
     }
@@ -209,7 +207,7 @@ void born_f32_fwd_kernel(typename std::conditional<PUR, PurArgs, FwdArgs>::type 
     const int T = p.T, D = p.D, BH = p.B * p.H;
     const int nmb = (T + kF32Rows - 1) / kF32Rows;
     const SplitMask m = {p.is_causal != 0, p.doc != nullptr, p.window};
-    const SplitBlock blk((int)blockIdx.x, (int)gridDim.x, BH, nmb, m.causal);
+    const SplitBlock blk((int)blockIdx.x, (int)gridDim.x, BH, nmb, m.causal, split_two_per_cu(sizeof(tiles)));
     const int b = blk.bh / p.H, h = blk.bh % p.H, m0 = blk.mb * kF32Rows;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -368,7 +366,7 @@ void born_f32_dq_kernel(typename std::conditional<PUR, PurArgs, BwdArgs>::type p
     const int T = p.T, D = p.D, BH = p.B * p.H;
     const int nmb = (T + kF32Rows - 1) / kF32Rows;
     const SplitMask m = {p.is_causal != 0, p.doc != nullptr, p.window};
-    const SplitBlock blk((int)blockIdx.x, (int)gridDim.x, BH, nmb, m.causal);
+    const SplitBlock blk((int)blockIdx.x, (int)gridDim.x, BH, nmb, m.causal, split_two_per_cu(sizeof(tiles)));
     const int b = blk.bh / p.H, h = blk.bh % p.H, m0 = blk.mb * kF32Rows;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -537,7 +535,7 @@ void born_f32_dkdv_kernel(typename std::conditional<PUR, PurArgs, BwdArgs>::type
     const int T = p.T, D = p.D, BH = p.B * p.H;
     const int nkb = (T + kF32Rows - 1) / kF32Rows;
     const SplitMask m = {p.is_causal != 0, p.doc != nullptr, p.window};
-    const SplitBlock blk((int)blockIdx.x, (int)gridDim.x, BH, nkb, false);
+    const SplitBlock blk((int)blockIdx.x, (int)gridDim.x, BH, nkb, false, split_two_per_cu(sizeof(tiles)));
     const int b = blk.bh / p.H, h = blk.bh % p.H, k0 = blk.mb * kF32Rows;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);

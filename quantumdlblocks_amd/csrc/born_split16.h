@@ -223,7 +223,7 @@ void born_split16_fwd_kernel(typename std::conditional<PUR, PurArgs, FwdArgs>::t
     const int T = p.T, D = p.D, BH = p.B * p.H;
     const int nmb = (T + BM - 1) / BM;
     const SplitMask m = {p.is_causal != 0, p.doc != nullptr, p.window};
-    const SplitBlock blk((int)blockIdx.x, (int)gridDim.x, BH, nmb, m.causal);
+    const SplitBlock blk((int)blockIdx.x, (int)gridDim.x, BH, nmb, m.causal, split_two_per_cu(C::SMEM));
     const int b = blk.bh / p.H, h = blk.bh % p.H, m0 = blk.mb * BM;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -426,7 +426,7 @@ void born_split16_dq_kernel(typename std::conditional<PUR, PurArgs, BwdArgs>::ty
     const int T = p.T, D = p.D, BH = p.B * p.H;
     const int nmb = (T + BM - 1) / BM;
     const SplitMask m = {p.is_causal != 0, p.doc != nullptr, p.window};
-    const SplitBlock blk((int)blockIdx.x, (int)gridDim.x, BH, nmb, m.causal);
+    const SplitBlock blk((int)blockIdx.x, (int)gridDim.x, BH, nmb, m.causal, split_two_per_cu(C::SMEM));
     const int b = blk.bh / p.H, h = blk.bh % p.H, m0 = blk.mb * BM;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -638,7 +638,7 @@ void born_split16_dkdv_kernel(typename std::conditional<PUR, PurArgs, BwdArgs>::
     const int T = p.T, D = p.D, BH = p.B * p.H;
     const int nkb = (T + 31) / 32;
     const SplitMask m = {p.is_causal != 0, p.doc != nullptr, p.window};
-    const SplitBlock blk((int)blockIdx.x, (int)gridDim.x, BH, nkb, false);
+    const SplitBlock blk((int)blockIdx.x, (int)gridDim.x, BH, nkb, false, split_two_per_cu(C::SMEM));
     const int b = blk.bh / p.H, h = blk.bh % p.H, k0 = blk.mb * 32;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);

@@ -87,6 +87,22 @@ constexpr bool split16_addressable(int64_t T) { return (T + 256) * 512 < ((int64
 constexpr uint32_t kSplitPastD = 0x7ffffff0u;
 constexpr uint32_t split16_load_at(uint32_t chunk, uint32_t tile) { return chunk + tile; }
 
+// Rank of workgroup `bid` among a launch's blocks, longest tile ranges first.
+// Where the whole launch is resident at once, two workgroups per CU (257 to
+// 512 of them), the second half goes out shortest first, so that a CU pairs a
+// long block with a short one (fp32 B2 H8 T1000 D64 step: 159 -> 142 us).
+// Where only one fits, the second half starts as the first half's blocks end,
+// and the longest of it must go first (causal, the pairing order and this one:
+// fp32 B1 H8 T2048 D128 forward 121.6 and 99.2 us, backward 406 and 336;
+// purified bf16 B1 H8 T4096 D128 forward 113.7 and 95.9; Born bf16 B1 H8 T2048
+// D96 backward 76.4 and 70.3).
+constexpr int split_rank(int bid, int grid, bool two_per_cu) {
+    return two_per_cu && grid <= 512 && bid >= 256 ? grid - 1 - (bid - 256) : bid;
+}
+// Whether two workgroups of that much tile memory fit the 160 KiB of a CU
+// (the rest of a workgroup's LDS is below 4 KiB).
+constexpr bool split_two_per_cu(int tile_bytes) { return 2 * (tile_bytes + 4 * 1024) <= 160 * 1024; }
+
 // bwd: dQ and dK/dV together (one side's row sums feed the other's kernel).
 template <class Args>
 inline bool split16_pays(const Args& a, bool bwd, bool pur) {

@@ -5,6 +5,7 @@ ends of the argument range."""
 
 from __future__ import annotations
 
+import heapq
 import os
 import shutil
 import subprocess
@@ -86,3 +87,41 @@ def test_offsets_of_chunks_past_the_head_dim(tmp_path):
         pytest.skip("no host compiler")
     (tmp_path / "offsets.cpp").write_text(OFFSETS)
     subprocess.run([gxx, "-std=c++17", "-fsyntax-only", str(tmp_path / "offsets.cpp")], check=True)
+
+
+ORDER = """
+#include <cstdio>
+#include <cstdlib>
+#include "%s"
+int main(int, char** v) {
+    const int grid = atoi(v[1]);
+    const bool two = qdl::split_two_per_cu(atoi(v[2]));
+    printf("%%d ", two);
+    for (int b = 0; b < grid; ++b) printf("%%d ", qdl::split_rank(b, grid, two));
+}
+""" % RULE
+
+
+@pytest.mark.parametrize("tile_kib,per_cu", [(16, 2), (32, 2), (64, 2), (96, 1), (128, 1)])
+def test_block_order_fits_the_workgroups_per_cu(tmp_path, tile_kib, per_cu):
+    """Causal B1 H8 T2048 in 32-row blocks: 512 workgroups of 1 .. 64 tiles on
+    256 CUs.  Where one fits a CU, each takes the next one as it ends, and an
+    order that is not longest first ends later; where two fit, all start at
+    once, the i-th and (i + 256)-th on one CU, and share its matrix pipes."""
+    gxx = shutil.which("g++")
+    if gxx is None:
+        pytest.skip("no host compiler")
+    (tmp_path / "order.cpp").write_text(ORDER)
+    subprocess.run([gxx, "-std=c++17", str(tmp_path / "order.cpp"), "-o", str(tmp_path / "order")], check=True)
+    got = subprocess.check_output([str(tmp_path / "order"), "512", str(tile_kib * 1024)], text=True).split()
+    two, rank = got[0] == "1", [int(r) for r in got[1:]]
+    assert two == (per_cu == 2) and sorted(rank) == list(range(512))
+    tiles = [64 - r // 8 for r in rank]
+    if two:
+        end = max(tiles[i] + tiles[i + 256] for i in range(256))
+    else:
+        free = [0] * 256
+        for t in tiles:
+            heapq.heapreplace(free, free[0] + t)
+        end = max(free)
+    assert end <= 65
