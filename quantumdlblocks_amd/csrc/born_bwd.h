@@ -710,7 +710,7 @@ void born_bwd_dkdv16_kernel(typename std::conditional<PUR, PurArgs, BwdArgs>::ty
 }
 
 // ---------------------------------------------------------------------------
-// dQ, fp32, D > 128 (v_mfma_f32_32x32x2_f32).  Same structure as the 16-bit kernel;
+// dQ, fp32, staged (v_mfma_f32_32x32x2_f32).  Same structure as the 16-bit kernel;
 // fp32 operands need no transposed copies: the contraction over keys reads
 // K[key][d] with d across lanes.
 // ---------------------------------------------------------------------------
@@ -900,31 +900,34 @@ void born_bwd_dq32_kernel(BwdArgs p) {
 }
 
 // ---------------------------------------------------------------------------
-// dK / dV, fp32, D > 128.  Keys stationary, one wave per workgroup; K' and V
-// rows of its 32 keys are B operands, read from an LDS copy.  Same
+// dK / dV, fp32, staged.  Keys stationary; K' and V rows of the wave's 32 keys are
+// B operands, in registers (KV_LDS = false) or, for wide heads, read from a
+// per-workgroup LDS copy (KV_LDS = true, one wave per workgroup).  Same
 // arithmetic as the 16-bit kernel; fp32 operands need no transposed copies.
 // CS column splits as in the 16-bit kernel: with CS == 2 two workgroups share
 // a key block, each accumulating dK, dV for half of the head dim's columns.
 // ---------------------------------------------------------------------------
-template <int DP, int BQ, int MODE, int CS = 1>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1)))
+template <int DP, int NW, int BQ, int MODE, bool KV_LDS, int CS = 1>
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void born_bwd_dkdv32_kernel(BwdArgs p) {
-    constexpr int BK = 32;
+    constexpr int BK = NW * 32;
     constexpr int KQ = DP / 8;
     constexpr int DBF = DP / 32;             // column blocks of the head dim
     constexpr int DB = (DBF + CS - 1) / CS;  // column blocks accumulated here (at most)
     constexpr int NQ = BQ / 32;
-    constexpr int NT = 64;
+    constexpr int NT = NW * 64;
     constexpr int RS = DP + 4;
+    constexpr int NBUF = KV_LDS ? 1 : 2;
     constexpr bool kDoc = (MODE == kGeneral);
     using Stage = RowStager32<BQ, DP, NT>;
+    static_assert(!KV_LDS || NW == 1, "LDS-resident K/V uses one wave per workgroup");
 
-    __shared__ __attribute__((aligned(16))) float q_lds[BQ * RS];
-    __shared__ __attribute__((aligned(16))) float d_lds[BQ * RS];
-    __shared__ __attribute__((aligned(16))) float kv_lds[2][32 * RS];
-    __shared__ __attribute__((aligned(16))) float nd_lds[BQ];
-    __shared__ __attribute__((aligned(16))) float zi_lds[BQ];
-    __shared__ __attribute__((aligned(16))) int32_t doc_lds[kDoc ? BQ : 1];
+    __shared__ __attribute__((aligned(16))) float q_lds[NBUF][BQ * RS];
+    __shared__ __attribute__((aligned(16))) float d_lds[NBUF][BQ * RS];
+    __shared__ __attribute__((aligned(16))) float kv_lds[KV_LDS ? 2 : 1][KV_LDS ? 32 * RS : 4];
+    __shared__ __attribute__((aligned(16))) float nd_lds[NBUF][BQ];
+    __shared__ __attribute__((aligned(16))) float zi_lds[NBUF][BQ];
+    __shared__ __attribute__((aligned(16))) int32_t doc_lds[kDoc ? NBUF : 1][kDoc ? BQ : 1];
     __shared__ int32_t span_red[kDoc ? 4 : 1];
 
     const int T = p.T, D = p.D;
@@ -959,16 +962,31 @@ void born_bwd_dkdv32_kernel(BwdArgs p) {
     const float sgn = (sc < 0.f) ? -1.f : 1.f;
 
     // B operands: K'[key][d(t, g)], V[key][d(t, g)] with d(t, g) = 8(t/4) + 4g + t%4.
-    for (int idx = tid; idx < 32 * (DP / 4); idx += NT) {
-        const int row = idx / (DP / 4), col = (idx % (DP / 4)) * 4;
-        const int kk = kw0 + row;
-        f32x4 x = {0.f, 0.f, 0.f, 0.f}, y = {0.f, 0.f, 0.f, 0.f};
-        if (kk < T && col < D) {
-            x = *reinterpret_cast<const f32x4*>(K + (size_t)kk * D + col) * sgn;
-            y = *reinterpret_cast<const f32x4*>(V + (size_t)kk * D + col);
+    f32x4 kr[KV_LDS ? 1 : KQ], vr[KV_LDS ? 1 : KQ];
+    if constexpr (KV_LDS) {
+        for (int idx = tid; idx < 32 * (DP / 4); idx += NT) {
+            const int row = idx / (DP / 4), col = (idx % (DP / 4)) * 4;
+            const int kk = kw0 + row;
+            f32x4 x = {0.f, 0.f, 0.f, 0.f}, y = {0.f, 0.f, 0.f, 0.f};
+            if (kk < T && col < D) {
+                x = *reinterpret_cast<const f32x4*>(K + (size_t)kk * D + col) * sgn;
+                y = *reinterpret_cast<const f32x4*>(V + (size_t)kk * D + col);
+            }
+            *reinterpret_cast<f32x4*>(&kv_lds[0][row * RS + col]) = x;
+            *reinterpret_cast<f32x4*>(&kv_lds[1][row * RS + col]) = y;
         }
-        *reinterpret_cast<f32x4*>(&kv_lds[0][row * RS + col]) = x;
-        *reinterpret_cast<f32x4*>(&kv_lds[1][row * RS + col]) = y;
+    } else {
+#pragma unroll
+        for (int u = 0; u < KQ; ++u) {
+            const int d = 8 * u + 4 * g;
+            f32x4 x = {0.f, 0.f, 0.f, 0.f}, y = {0.f, 0.f, 0.f, 0.f};
+            if (key < T && d < D) {
+                x = *reinterpret_cast<const f32x4*>(K + (size_t)key * D + d);
+                y = *reinterpret_cast<const f32x4*>(V + (size_t)key * D + d);
+            }
+            kr[u] = x * sgn;
+            vr[u] = y;
+        }
     }
     const int kdoc = (has_doc && key < T) ? docb[key] : -2;
 
@@ -990,13 +1008,13 @@ void born_bwd_dkdv32_kernel(BwdArgs p) {
             if (kDoc && has_doc) dreg = i < T ? docb[i] : -1;
         }
     };
-    auto store_tile = [&]() {
-        qst.template store_rows<RS>(q_lds, tid);
-        dst.template store_rows<RS>(d_lds, tid);
+    auto store_tile = [&](int buf) {
+        qst.template store_rows<RS>(q_lds[buf], tid);
+        dst.template store_rows<RS>(d_lds[buf], tid);
         if (tid < BQ) {
-            nd_lds[tid] = ndreg;
-            zi_lds[tid] = zireg;
-            if (kDoc && has_doc) doc_lds[tid] = dreg;
+            nd_lds[buf][tid] = ndreg;
+            zi_lds[buf][tid] = zireg;
+            if (kDoc && has_doc) doc_lds[buf][tid] = dreg;
         }
     };
 
@@ -1030,17 +1048,19 @@ void born_bwd_dkdv32_kernel(BwdArgs p) {
     }
     if (ntiles > 0) {
         if (!first_issued) load_tile(q_lo);
-        store_tile();
+        store_tile(0);
     }
     __syncthreads();
 
     for (int t = 0; t < ntiles; ++t) {
         const int i0 = q_lo + t * BQ;
+        const int buf = (NBUF == 2) ? (t & 1) : 0;
         const bool more = (t + 1) < ntiles;
+        if (NBUF == 2 && more) load_tile(i0 + BQ);
 
         bool active = kw0 < T;
         bool need_mask = false;
-        if constexpr (kDoc) need_mask = has_doc && !one_document(doc_lds, BQ, kdoc, kdoc);
+        if constexpr (kDoc) need_mask = has_doc && !one_document(doc_lds[buf], BQ, kdoc, kdoc);
         if (causal) {
             active = active && (i0 + BQ - 1 >= kw0);
             need_mask = need_mask || (i0 < kw0 + 31);
@@ -1055,8 +1075,8 @@ void born_bwd_dkdv32_kernel(BwdArgs p) {
                 f32x16 s = zero16(), dp, zi;
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    const f32x4 n4 = *reinterpret_cast<const f32x4*>(&nd_lds[qs * 32 + 8 * j + 4 * g]);
-                    const f32x4 z4 = *reinterpret_cast<const f32x4*>(&zi_lds[qs * 32 + 8 * j + 4 * g]);
+                    const f32x4 n4 = *reinterpret_cast<const f32x4*>(&nd_lds[buf][qs * 32 + 8 * j + 4 * g]);
+                    const f32x4 z4 = *reinterpret_cast<const f32x4*>(&zi_lds[buf][qs * 32 + 8 * j + 4 * g]);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         dp[4 * j + e] = n4[e];
@@ -1065,10 +1085,16 @@ void born_bwd_dkdv32_kernel(BwdArgs p) {
                 }
 #pragma unroll
                 for (int u = 0; u < KQ; ++u) {
-                    const f32x4 aq = *reinterpret_cast<const f32x4*>(&q_lds[(qs * 32 + c) * RS + 8 * u + 4 * g]);
-                    const f32x4 ad = *reinterpret_cast<const f32x4*>(&d_lds[(qs * 32 + c) * RS + 8 * u + 4 * g]);
-                    const f32x4 bk = *reinterpret_cast<const f32x4*>(&kv_lds[0][c * RS + 8 * u + 4 * g]);
-                    const f32x4 bv = *reinterpret_cast<const f32x4*>(&kv_lds[1][c * RS + 8 * u + 4 * g]);
+                    const f32x4 aq = *reinterpret_cast<const f32x4*>(&q_lds[buf][(qs * 32 + c) * RS + 8 * u + 4 * g]);
+                    const f32x4 ad = *reinterpret_cast<const f32x4*>(&d_lds[buf][(qs * 32 + c) * RS + 8 * u + 4 * g]);
+                    f32x4 bk, bv;
+                    if constexpr (KV_LDS) {
+                        bk = *reinterpret_cast<const f32x4*>(&kv_lds[0][c * RS + 8 * u + 4 * g]);
+                        bv = *reinterpret_cast<const f32x4*>(&kv_lds[1][c * RS + 8 * u + 4 * g]);
+                    } else {
+                        bk = kr[u];
+                        bv = vr[u];
+                    }
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         s = mfma_f32(aq[e], bk[e], s);
@@ -1082,7 +1108,7 @@ void born_bwd_dkdv32_kernel(BwdArgs p) {
                     float a = fmaxf(s[r], 0.f);
                     if (need_mask) {
                         const int qi = ibase + 8 * (r >> 2) + (r & 3);
-                        const int qd = (kDoc && has_doc) ? doc_lds[qi - i0] : 0;
+                        const int qd = (kDoc && has_doc) ? doc_lds[buf][qi - i0] : 0;
                         if (!visible<MODE>(qi, key, causal, window, has_doc, qd, kdoc)) a = 0.f;
                     }
                     const float t = a * zi[r];
@@ -1095,18 +1121,23 @@ void born_bwd_dkdv32_kernel(BwdArgs p) {
 #pragma unroll
                     for (int db = 0; db < DB; ++db) {
                         if (DBF % CS != 0 && db0 + db >= DBF) break;  // the last split's short share
-                        dv[db] = mfma_f32(d_lds[qrow * RS + (db0 + db) * 32 + c], w[r], dv[db]);
-                        dk[db] = mfma_f32(q_lds[qrow * RS + (db0 + db) * 32 + c], uu[r], dk[db]);
+                        dv[db] = mfma_f32(d_lds[buf][qrow * RS + (db0 + db) * 32 + c], w[r], dv[db]);
+                        dk[db] = mfma_f32(q_lds[buf][qrow * RS + (db0 + db) * 32 + c], uu[r], dk[db]);
                     }
                 }
             }
         }
-        __syncthreads();
-        if (more) {
-            load_tile(i0 + BQ);
-            store_tile();
+        if (NBUF == 2) {
+            if (more) store_tile(buf ^ 1);
+            __syncthreads();
+        } else {
+            __syncthreads();
+            if (more) {
+                load_tile(i0 + BQ);
+                store_tile(0);
+            }
+            __syncthreads();
         }
-        __syncthreads();
     }
 
     if (key < T) {
@@ -1149,9 +1180,12 @@ struct Bwd16Cfg {
     static constexpr int NW = 4;
 };
 
-// fp32 above D = 128 (up to there: born_f32.h).
+// fp32: head dims above 128, and the launches of f32_staged at padded head dim
+// 128 (f32_rule.h; the others up to there: born_f32.h).
 template <int DP>
 struct Bwd32Cfg {
+    static constexpr bool KV_LDS = DP > 128;
+    static constexpr int KV_NW = KV_LDS ? 1 : 4;
     // dK/dV column splits: dense launches at D = 192 and 256 (each split
     // forms S and dP again, which outweighs the spills it removes elsewhere:
     // B4 H2 T2048 backward D = 256 dense 6917 -> 5034 us, D = 192 dense
@@ -1317,9 +1351,11 @@ hipError_t launch_bwd32(const BwdArgs& a, hipStream_t st) {
     if (e != hipSuccess) return e;
     const unsigned BH = (unsigned)(a.B * a.H);
     {
+        constexpr int BK = C::KV_NW * 32;
         constexpr int CS = C::template kv_cs<MODE>();
-        const dim3 grid((unsigned)((a.T + 31) / 32) * BH * CS);
-        hipLaunchKernelGGL((born_bwd_dkdv32_kernel<DP, C::BQ, MODE, CS>), grid, dim3(64), 0, st, a);
+        const dim3 grid((unsigned)((a.T + BK - 1) / BK) * BH * CS);
+        hipLaunchKernelGGL((born_bwd_dkdv32_kernel<DP, C::KV_NW, C::BQ, MODE, C::KV_LDS, CS>), grid,
+                           dim3(C::KV_NW * 64), 0, st, a);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     {

@@ -1,5 +1,5 @@
-// fp32 flash-Born and purified-Born attention for head dims up to 128:
-// forward, dQ and dK/dV on v_mfma_f32_32x32x2_f32 (the reference runs its
+// fp32 flash-Born and purified-Born attention for head dims up to 128 (but for
+// the launches of f32_staged): forward, dQ and dK/dV on v_mfma_f32_32x32x2_f32 (the reference runs its
 // fp32 dots with allow_tf32=False, flash_born.py:160, 298).
 //
 // What bounds it: the fp32 matrix pipe (64 cycles per 32x32x2 MFMA, 153
@@ -42,13 +42,11 @@
 
 #include "born_common.h"
 #include "born_fwd_fast.h"
+#include "f32_rule.h"
 #include "purified_args.h"
 #include "split16_rule.h"
 
 namespace qdl {
-
-constexpr int kF32MaxD = 128;  // wider heads take the staged kernels (born_fwd.h, born_bwd.h, purified.h)
-constexpr int kF32Rows = 32;   // stationary rows per workgroup
 
 // A descriptor over the 32 rows from r0 (uniform) of a slice of `width` floats
 // per row; loads past row T return zeros.
@@ -688,22 +686,7 @@ void born_f32_dkdv_kernel(typename std::conditional<PUR, PurArgs, BwdArgs>::type
     f32_reduce_store<DB, NW>(red, reinterpret_cast<float*>(p.dk) + base, k0, T, D, [&](int, f32x4 x) -> f32x4 { return x * fk; });
 }
 
-inline int f32_groups(int B, int H, int T) { return (T + kF32Rows - 1) / kF32Rows * B * H; }
-
-// Waves per workgroup: four, unless the blocks are many for their length.  One
-// wave per block does without the reduction and the idle waves of short
-// blocks, but its launch ends with whole blocks; the two cross between 128 and
-// 205 blocks per tile of the mean block.  Steps measured with one wave and
-// with four: B16 H16 T512 D32 (482) 241 and 290 us, B16 H16 T256 D128 (455) 322
-// and 532, B4 H8 T1024 D32 with a 128-key window (205) 68 and 82; B8 H16 T300
-// D96 dense (128) 374 and 351, B8 H8 T1024 D64 (124) 513 and 446, B4 H8 T512
-// D64 (60) 195 and 94.
-inline int f32_waves(int B, int H, int T, bool causal, int window) {
-    const int64_t tiles = (T + kF32Rows - 1) / kF32Rows;
-    int64_t mean = causal ? (tiles + 1) / 2 : tiles;
-    if (causal && window > 0 && window / kF32Rows + 1 < mean) mean = window / kF32Rows + 1;
-    return (int64_t)f32_groups(B, H, T) >= 160 * mean ? 1 : 4;
-}
+inline int f32_groups(int B, int H, int T) { return (int)f32_blocks((int64_t)B * H, T); }
 
 #define QDL_F32_DP(D, BODY)                          \
     switch (((D) + 31) / 32) {                       \
@@ -722,7 +705,7 @@ inline int f32_waves(int B, int H, int T, bool causal, int window) {
 template <bool PUR, class Args>
 hipError_t launch_f32_fwd(const Args& a, hipStream_t st) {
     const dim3 grid((unsigned)f32_groups(a.B, a.H, a.T));
-    const int nw = f32_waves(a.B, a.H, a.T, a.is_causal != 0, a.window);
+    const int nw = f32_waves((int64_t)a.B * a.H, a.T, a.D, a.is_causal != 0, a.window);
     QDL_F32_DP(a.D, {
         QDL_F32_NW(nw, {
             hipLaunchKernelGGL((born_f32_fwd_kernel<DPV, PUR, NWV>), grid, dim3(64 * NWV), 0, st, a);
@@ -735,7 +718,7 @@ hipError_t launch_f32_fwd(const Args& a, hipStream_t st) {
 template <bool PUR, class Args>
 hipError_t launch_f32_bwd(const Args& a, hipStream_t st) {
     const dim3 grid((unsigned)f32_groups(a.B, a.H, a.T));
-    const int nw = f32_waves(a.B, a.H, a.T, a.is_causal != 0, a.window);
+    const int nw = f32_waves((int64_t)a.B * a.H, a.T, a.D, a.is_causal != 0, a.window);
     QDL_F32_DP(a.D, {
         QDL_F32_NW(nw, {
             hipLaunchKernelGGL((born_f32_dq_kernel<DPV, PUR, NWV>), grid, dim3(64 * NWV), 0, st, a);

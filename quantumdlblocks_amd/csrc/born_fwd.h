@@ -485,8 +485,10 @@ void born_fwd16_kernel(typename std::conditional<PUR, PurArgs, FwdArgs>::type p)
 }
 
 // ---------------------------------------------------------------------------
-// fp32 forward above D = 128 (up to there: born_f32.h): v_mfma_f32_32x32x2_f32, no reduced-precision operands
-// (the reference runs its fp32 dots with allow_tf32=False).
+// fp32 forward above D = 128, and the launches of f32_staged at padded head
+// dims 96 and 128 (f32_rule.h; the others up to there: born_f32.h):
+// v_mfma_f32_32x32x2_f32, no reduced-precision operands (the reference runs
+// its fp32 dots with allow_tf32=False).
 // ---------------------------------------------------------------------------
 template <int DP, int NW, int BN, int MODE, int WPE>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
@@ -716,7 +718,7 @@ template <int DP>
 struct Fwd32Cfg {
     static constexpr int NW = 4;
     static constexpr int BN = 32;
-    static constexpr int WPE = 1;
+    static constexpr int WPE = DP <= 128 ? 2 : 1;
     static constexpr int BM = NW * 32;
 };
 

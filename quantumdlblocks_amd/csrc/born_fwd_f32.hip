@@ -7,9 +7,13 @@
 namespace qdl {
 
 hipError_t fwd_launch_f32(const FwdArgs& a, hipStream_t s) {
-    if (a.D <= kF32MaxD) return launch_f32_fwd<false>(a, s);
+    if (!f32_staged(false, false, (int64_t)a.B * a.H, a.T, a.D, a.is_causal != 0, a.window,
+                    a.doc != nullptr))
+        return launch_f32_fwd<false>(a, s);
     const int dp = padded_head_dim(a.D);
     const int mode = mask_mode(a.is_causal, a.window, a.doc);
+    if (dp == 96) return mode == kDense ? launch_fwd32<96, kDense>(a, s) : launch_fwd32<96, kGeneral>(a, s);
+    if (dp == 128) return mode == kDense ? launch_fwd32<128, kDense>(a, s) : launch_fwd32<128, kGeneral>(a, s);
 #define QDL_MODE_BODY(M) return launch_fwd32<DPV, M>(a, s);
 #define QDL_DP_BODY(D_) { constexpr int DPV = D_; QDL_SWITCH_MODE(mode, QDL_MODE_BODY) }
     QDL_SWITCH_DP_WIDE(dp, QDL_DP_BODY)

@@ -88,7 +88,10 @@ static hipError_t purified_bwd_dispatch(const PurArgs& a, hipStream_t s) {
         return launch_purified_param_reduce(a, nwg, s);
     }
     if (k16 && (a.D > 128 || a.doc != nullptr)) return purified_wide_bwd_launch(E::kDtype, a, s);
-    if (!k16 && a.D <= kF32MaxD && purified_split_ok<IN>(a)) return purified_bwd_f32_launch(a, s);
+    if (!k16 && purified_split_ok<IN>(a) &&
+        !f32_staged(true, true, (int64_t)a.B * a.H, a.T, a.D, a.is_causal != 0, a.window,
+                    a.doc != nullptr))
+        return purified_bwd_f32_launch(a, s);
     switch (purified_padded_dim(a.D)) {
         case 32: return launch_purified_bwd<IN, 32>(a, s);
         case 64: return launch_purified_bwd<IN, 64>(a, s);

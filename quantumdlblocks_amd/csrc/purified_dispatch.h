@@ -30,7 +30,7 @@ inline bool purified_split_ok(const PurArgs& a) {
     return std::is_same<IN, BF16>::value || !a.param_grads;
 }
 
-// fp32 inputs up to D = 128 (born_fwd_f32.hip, born_bwd_f32.hip).
+// fp32 inputs up to D = 128 but for f32_staged (born_fwd_f32.hip, born_bwd_f32.hip).
 hipError_t purified_fwd_f32_launch(const PurArgs& a, hipStream_t s);
 hipError_t purified_bwd_f32_launch(const PurArgs& a, hipStream_t s);
 

@@ -68,7 +68,10 @@ static hipError_t purified_fwd_dispatch(const PurArgs& a, hipStream_t s) {
     // 16-bit-MFMA kernels' purified mode.
     if (k16 && purified_d256_ok(a)) return purified_fwd_d256_launch(E::kDtype, a, s);
     if (k16 && (a.D > 128 || a.doc != nullptr)) return purified_wide_fwd_launch(E::kDtype, a, s);
-    if (!k16 && a.D <= kF32MaxD && purified_split_ok<IN>(a)) return purified_fwd_f32_launch(a, s);
+    if (!k16 && purified_split_ok<IN>(a) &&
+        !f32_staged(true, false, (int64_t)a.B * a.H, a.T, a.D, a.is_causal != 0, a.window,
+                    a.doc != nullptr))
+        return purified_fwd_f32_launch(a, s);
     switch (purified_padded_dim(a.D)) {
         case 32: return launch_purified_fwd<IN, 32>(a, s);
         case 64: return launch_purified_fwd<IN, 64>(a, s);

@@ -118,3 +118,12 @@ def test_f32_many_short_heads(cuda_device, mask, purified):
     """512 blocks of up to four tiles: one wave per block, and the launch
     whose second half goes out in the opposite order."""
     _case(64, 97, 40, mask, purified, cuda_device)
+
+
+@pytest.mark.parametrize("purified", [False, True], ids=["born", "purified"])
+@pytest.mark.parametrize("mask", ["dense", "window_nc", "docs_dense"])
+@pytest.mark.parametrize("D", [72, 96, 104, 128])
+def test_f32_full_chip_without_causality(cuda_device, D, mask, purified):
+    """512 blocks of 128 rows (f32_staged, test_f32_rule.py): the staged
+    kernels at these head dims, forward and backward or one of them."""
+    _case(256, 129, D, mask, purified, cuda_device)
