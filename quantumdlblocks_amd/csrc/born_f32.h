@@ -134,6 +134,12 @@ struct SplitBlock {
     }
 };
 
+// Document of a block's own row; past T the last row's.  Those rows are not
+// stored and add nothing, but an id of their own would send every tile of the
+// last block through the masked body (Born bf16 B1 H4 T1300 D128 dense, one document:
+// forward 46.2 -> 29.4 us, backward 94 -> 68).
+__device__ __forceinline__ int split_row_doc(const int32_t* docb, int row, int T) { return docb[min(row, T - 1)]; }
+
 // Which (query, key) pairs a block's rows see.
 struct SplitMask {
     bool causal, has_doc;
@@ -227,7 +233,7 @@ void born_f32_fwd_kernel(typename std::conditional<PUR, PurArgs, FwdArgs>::type 
         t_lo = __builtin_amdgcn_readfirstlane(sp.x);
         t_hi = __builtin_amdgcn_readfirstlane(sp.y);
     }
-    const int qdoc = (m.has_doc && qi < T) ? docb[qi] : -1;
+    const int qdoc = m.has_doc ? split_row_doc(docb, qi, T) : -1;
 
     f32x4 qr[KQ];
     f32_load_rows(qr, Q, qi, T, D, g);
@@ -396,7 +402,7 @@ void born_f32_dq_kernel(typename std::conditional<PUR, PurArgs, BwdArgs>::type p
         t_lo = __builtin_amdgcn_readfirstlane(sp.x);
         t_hi = __builtin_amdgcn_readfirstlane(sp.y);
     }
-    const int qdoc = (m.has_doc && qi < T) ? docb[qi] : -1;
+    const int qdoc = m.has_doc ? split_row_doc(docb, qi, T) : -1;
 
     f32x4 qr[KQ], dr[KQ];
     f32_load_rows(qr, Q, qi, T, D, g);
@@ -558,7 +564,7 @@ void born_f32_dkdv_kernel(typename std::conditional<PUR, PurArgs, BwdArgs>::type
         t_lo = __builtin_amdgcn_readfirstlane(sp.x);
         t_hi = __builtin_amdgcn_readfirstlane(sp.y);
     }
-    const int kdoc = (m.has_doc && key < T) ? docb[key] : -2;
+    const int kdoc = m.has_doc ? split_row_doc(docb, key, T) : -2;
 
     f32x4 kr[KQ], vr[KQ];
     f32_load_rows(kr, K, key, T, D, g);

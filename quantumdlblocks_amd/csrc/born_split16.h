@@ -277,7 +277,7 @@ void born_split16_fwd_kernel(typename std::conditional<PUR, PurArgs, FwdArgs>::t
     for (int qb = 0; qb < NQB; ++qb) {
         const int qi = m0 + 32 * qb + c;
         split_load_rows(qr[qb], Q, qi, T, D, g);
-        qdoc[qb] = (m.has_doc && qi < T) ? docb[qi] : -1;
+        qdoc[qb] = m.has_doc ? split_row_doc(docb, qi, T) : -1;
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) qr[qb][ks] ^= flip;
 #pragma unroll
@@ -483,7 +483,7 @@ void born_split16_dq_kernel(typename std::conditional<PUR, PurArgs, BwdArgs>::ty
         const bool ok = qi < T;
         split_load_rows(qr[qb], Q, qi, T, D, g);
         split_load_rows(dr[qb], dO, qi, T, D, g);
-        qdoc[qb] = (m.has_doc && ok) ? docb[qi] : -1;
+        qdoc[qb] = m.has_doc ? split_row_doc(docb, qi, T) : -1;
         // delta = dO . O of the row (each half wave holds half of it).
         float dl = 0.f;
 #pragma unroll
@@ -697,7 +697,7 @@ void born_split16_dkdv_kernel(typename std::conditional<PUR, PurArgs, BwdArgs>::
     u32x4 kr[KS], vr[KS];
     split_load_rows(kr, K, key, T, D, g);
     split_load_rows(vr, V, key, T, D, g);
-    int kdoc = (m.has_doc && key < T) ? docb[key] : -2;
+    int kdoc = m.has_doc ? split_row_doc(docb, key, T) : -2;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
         kr[ks] ^= flip;

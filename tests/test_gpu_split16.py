@@ -78,6 +78,15 @@ def test_unsorted_documents(cuda_device, purified):
     _case(2, 2, 600, 64, torch.bfloat16, "docs", purified, cuda_device, sorted_docs=False)
 
 
+@pytest.mark.parametrize("purified", [False, True], ids=["born", "purified"])
+@pytest.mark.parametrize("mask", ["docs", "docs_dense"])
+@pytest.mark.parametrize("B,T", [(1, 1301), (2, 705), (2, 1027)])
+def test_documents_of_ragged_length(cuda_device, B, T, mask, purified):
+    """A last block of few rows, ids partly out of range, and a second batch
+    whose ids start at 4 bytes past a 16-byte boundary."""
+    _case(B, 2, T, 64, torch.bfloat16, mask, purified, cuda_device)
+
+
 @pytest.mark.parametrize("H", [8, 16])
 def test_two_workgroups_per_cu(cuda_device, H):
     """257 to 512 workgroups: the second half goes out in the opposite order."""
