@@ -1,9 +1,10 @@
 """16-bit attention of few blocks on the wave-split kernels (born_split16.h):
-32 or 64 stationary rows per workgroup, every fourth 32-row tile per wave.
-Shapes few enough for those kernels (split16_rule.h; test_split16_rule.py), at the edges of their blocks and tiles, for every padded head dim, mask
-and both 16-bit types.  Bounds: those of the forward, backward and purified
-tests (2e-2 of the largest value for 16-bit outputs, their floors for
-gradients that cancel).
+32 or 64 stationary rows per workgroup, every fourth 32-row tile per wave.  The
+shapes are lists of test_split16_rule.py, which asserts on the host that each
+takes those kernels: at the edges of their blocks and tiles, for every padded
+head dim, mask and both 16-bit types.  Bounds: those of the forward, backward
+and purified tests (2e-2 of the largest value for 16-bit outputs, their floors
+for gradients that cancel).
 """
 
 from __future__ import annotations
@@ -16,20 +17,11 @@ from oracle import born_oracle as orc
 from test_gpu_backward import _check_bwd
 from test_gpu_f32 import check_pur_fixed
 from test_gpu_purified import _check_pur
-from util import TOL, f64, rel_err, seeded_inputs
+from test_split16_rule import (FULL_CHIP, FULL_CHIP_PURIFIED, HEAD_DIMS, LENGTHS, MASKS, RAGGED_DOCS, UNSORTED_DOCS,
+                               WINDOW_NC_D128)
+from util import TOL, f64, seeded_inputs
 
 pytestmark = pytest.mark.gpu
-
-MASKS = {
-    "causal": (True, 0, False),
-    "dense": (False, 0, False),
-    "window": (True, 300, False),
-    "window_nc": (False, 300, False),
-    "docs": (True, 0, True),
-    "docs_window": (True, 300, True),
-    "docs_dense": (False, 0, True),
-}
-
 
 def _case(B, H, T, D, dtype, mask, purified, device, sorted_docs=True):
     causal, window, docs = MASKS[mask]
@@ -52,42 +44,45 @@ def _case(B, H, T, D, dtype, mask, purified, device, sorted_docs=True):
 
     doc_t = None if doc is None else torch.as_tensor(doc, dtype=torch.int32, device=device)
     out = flash_born_attention(q, k, v, torch.tensor(scale, device=device), doc_ids=doc_t, **kw)
-    ref, _ = orc.forward(f64(q), f64(k), f64(v), np.asarray(scale), causal, 1e-12, window, doc)
-    assert rel_err(f64(out), ref) <= TOL[dtype]
+    ref, z = orc.forward(f64(q), f64(k), f64(v), np.asarray(scale), causal, 1e-12, window, doc)
+    bound = TOL[dtype] * np.abs(ref).max()
+    if dtype == torch.float16:
+        # The weights of P.V are rounded to fp16, as the reference's are
+        # (flash_born.py:183): by at most 2^-25 each below its normal range,
+        # which a document's first rows, of one or two keys, can show.
+        seen = orc.visible_mask(T, causal, window, doc).astype(np.float64)
+        bound = bound + 2.0 ** -25 * (seen @ np.abs(f64(v))) / z[..., None]
+    assert (np.abs(f64(out) - ref) <= bound).all()
     _check_bwd(B, H, T, D, dtype, device, scale=scale, doc=doc, std=0.5, seed=T + D, check_dscale=mask == "dense", **kw)
 
 
 @pytest.mark.parametrize("purified", [False, True], ids=["born", "purified"])
-@pytest.mark.parametrize("mask", list(MASKS))
-@pytest.mark.parametrize("D", [24, 64, 72, 96, 120, 128, 160, 256])
+@pytest.mark.parametrize("case", HEAD_DIMS, ids=str)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=str)
-def test_masks_and_head_dims(cuda_device, D, mask, purified, dtype):
-    _case(1, 2, 700, D, dtype, mask, purified, cuda_device)
+def test_masks_and_head_dims(cuda_device, case, purified, dtype):
+    B, H, T, D, mask = case
+    _case(B, H, T, D, dtype, mask, purified, cuda_device)
 
 
 @pytest.mark.parametrize("purified", [False, True], ids=["born", "purified"])
-@pytest.mark.parametrize("T", [384, 415, 416, 417, 447, 448, 449, 513, 1000])
-@pytest.mark.parametrize("D", [64, 128])
-def test_lengths(cuda_device, T, D, purified):
-    for mask in ("causal", "dense"):
-        _case(1, 3, T, D, torch.bfloat16, mask, purified, cuda_device)
+@pytest.mark.parametrize("case", LENGTHS + WINDOW_NC_D128 + RAGGED_DOCS, ids=str)
+def test_lengths(cuda_device, case, purified):
+    """Block and tile edges; with documents also ids partly out of range, and a
+    second batch whose ids start 4 bytes past a 16-byte boundary."""
+    B, H, T, D, mask = case
+    _case(B, H, T, D, torch.bfloat16, mask, purified, cuda_device)
 
 
 @pytest.mark.parametrize("purified", [False, True], ids=["born", "purified"])
 def test_unsorted_documents(cuda_device, purified):
-    _case(2, 2, 600, 64, torch.bfloat16, "docs", purified, cuda_device, sorted_docs=False)
+    for B, H, T, D, mask in UNSORTED_DOCS:
+        _case(B, H, T, D, torch.bfloat16, mask, purified, cuda_device, sorted_docs=False)
 
 
-@pytest.mark.parametrize("purified", [False, True], ids=["born", "purified"])
-@pytest.mark.parametrize("mask", ["docs", "docs_dense"])
-@pytest.mark.parametrize("B,T", [(1, 1301), (2, 705), (2, 1027)])
-def test_documents_of_ragged_length(cuda_device, B, T, mask, purified):
-    """A last block of few rows, ids partly out of range, and a second batch
-    whose ids start at 4 bytes past a 16-byte boundary."""
-    _case(B, 2, T, 64, torch.bfloat16, mask, purified, cuda_device)
-
-
-@pytest.mark.parametrize("H", [8, 16])
-def test_two_workgroups_per_cu(cuda_device, H):
-    """257 to 512 workgroups: the second half goes out in the opposite order."""
-    _case(2, H, 1100, 64, torch.bfloat16, "causal", False, cuda_device)
+@pytest.mark.parametrize("purified,case", [(False, c) for c in FULL_CHIP] +
+                         [(True, c) for c in FULL_CHIP + FULL_CHIP_PURIFIED], ids=str)
+def test_full_chip(cuda_device, purified, case):
+    """257 to 512 workgroups: where two fit a CU the second half goes out in the
+    opposite order."""
+    B, H, T, D, mask = case
+    _case(B, H, T, D, torch.bfloat16, mask, purified, cuda_device)

@@ -1,7 +1,7 @@
 """The rule that sends a 16-bit launch of few blocks to the wave-split kernels
-(csrc/split16_rule.h), compiled on the host: it takes the shapes their GPU
-tests use, leaves the tuned kernels' own ranges alone, and stays finite at the
-ends of the argument range."""
+(csrc/split16_rule.h), compiled on the host: it takes each launch of their GPU
+tests (test_gpu_split16.py, from the same lists), leaves the tuned kernels' own
+ranges alone, and stays finite at the ends of the argument range."""
 
 from __future__ import annotations
 
@@ -12,15 +12,40 @@ import subprocess
 
 import pytest
 
+# name: (causal, window, documents)
+MASKS = {
+    "causal": (True, 0, False),
+    "dense": (False, 0, False),
+    "window": (True, 300, False),
+    "window_nc": (False, 300, False),
+    "docs": (True, 0, True),
+    "docs_window": (True, 300, True),
+    "docs_dense": (False, 0, True),
+}
+# What test_gpu_split16.py runs, as (B, H, T, D, mask).
+HEAD_DIMS = [(1, 2, 1000, D, mask) for D in (24, 64, 72, 96, 120, 128, 160, 256) for mask in MASKS]
+LENGTHS = [(1, 3, T, D, mask) for D, lengths in ((64, (449, 479, 480, 481, 512, 513, 1000)),
+                                                 (128, (735, 736, 737, 767, 768, 833, 1000)))
+           for T in lengths for mask in ("causal", "dense")]
+WINDOW_NC_D128 = [(1, 2, 1500, D, "window_nc") for D in (120, 128)]
+RAGGED_DOCS = [(B, 2, T, 64, mask) for B, T in ((1, 1301), (2, 705), (2, 1027)) for mask in ("docs", "docs_dense")]
+UNSORTED_DOCS = [(2, 2, 600, 64, "docs")]
+# 257 to 512 workgroups in some kernel: dK/dV (32-row blocks) or the forward and
+# dQ (64-row ones), where two fit a CU (padded head dim 64) and where one does.
+FULL_CHIP = [(1, 8, 1100, 64, "causal"), (2, 8, 1100, 64, "causal"), (2, 6, 1100, 96, "causal"),
+             (1, 8, 1200, 128, "causal"), (1, 8, 1100, 160, "causal")]
+FULL_CHIP_PURIFIED = [(2, 6, 1500, 96, "causal")]  # the Born forward of this one is a tuned kernel's
+
 RULE = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "quantumdlblocks_amd", "csrc",
                     "split16_rule.h")
 MAIN = """
 #include <cstdio>
 #include <cstdlib>
 #include "%s"
-struct A { int B, H, T, D, is_causal, window; };
+struct A { int B, H, T, D, is_causal, window; const int* doc; };
 int main(int, char** v) {
-    const A a = {atoi(v[1]), atoi(v[2]), atoi(v[3]), atoi(v[4]), atoi(v[5]), atoi(v[6])};
+    const int id = 0;
+    const A a = {atoi(v[1]), atoi(v[2]), atoi(v[3]), atoi(v[4]), atoi(v[5]), atoi(v[6]), atoi(v[7]) ? &id : nullptr};
     for (int pur = 0; pur < 2; ++pur)
         printf("%%d %%d ", qdl::split16_pays(a, false, pur), qdl::split16_pays(a, true, pur));
 }
@@ -36,20 +61,31 @@ def rule(tmp_path_factory):
     (d / "main.cpp").write_text(MAIN)
     subprocess.run([gxx, "-std=c++17", str(d / "main.cpp"), "-o", str(d / "rule")], check=True)
 
-    def ask(B, H, T, D, causal=1, window=0):
-        """(Born forward, Born backward, purified forward, purified backward)"""
-        args = [str(x) for x in (B, H, T, D, causal, window)]
+    def ask(B, H, T, D, mask="causal"):
+        """[Born forward, Born backward, purified forward, purified backward]"""
+        args = [str(int(x)) for x in (B, H, T, D, *MASKS[mask])]
         return [w == "1" for w in subprocess.check_output([str(d / "rule"), *args], text=True).split()]
 
     return ask
 
 
-@pytest.mark.parametrize("D", [24, 64, 72, 96, 120, 128, 160, 256])
-@pytest.mark.parametrize("causal,window", [(1, 0), (0, 0), (0, 300)])
-def test_few_blocks_take_the_split_kernels(rule, D, causal, window):
-    assert any(rule(1, 2, 700, D, causal, window))
-    if window == 0:
-        assert all(rule(1, 2, 1000, D, causal, window))
+@pytest.mark.parametrize("case", HEAD_DIMS, ids=str)
+def test_every_head_dim_and_mask_takes_the_split_kernels(rule, case):
+    """All four passes, but the Born forward at padded head dims 96 and 128
+    with a window (too few tiles a block at this length)."""
+    B, H, T, D, mask = case
+    born_fwd = D <= 64 or D > 128 or not MASKS[mask][1]
+    assert rule(*case) == [born_fwd, True, True, True]
+
+
+@pytest.mark.parametrize("case", LENGTHS + WINDOW_NC_D128 + RAGGED_DOCS + UNSORTED_DOCS + FULL_CHIP, ids=str)
+def test_launches_that_take_the_split_kernels_in_every_pass(rule, case):
+    assert rule(*case) == [True] * 4
+
+
+def test_full_chip_of_purified_blocks(rule):
+    for case in FULL_CHIP_PURIFIED:
+        assert rule(*case) == [False, True, True, True]
 
 
 @pytest.mark.parametrize("B,H,T,D", [(16, 16, 1024, 64), (16, 16, 2048, 64), (32, 4, 1024, 64), (16, 8, 2048, 128),
