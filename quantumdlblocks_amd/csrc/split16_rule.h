@@ -49,9 +49,9 @@ constexpr SplitCost kSplitCost[2][5][3] = {
      {{4.8, 2.25, 11.0, 2.00, 5.2}, {10.2, 2.19, 14.6, 2.20, 4.3}, {7.3, 2.54, 7.3, 1.93, 6.1}},
      {{7.4, 2.60, 10.0, 2.00, 8.0}, {11.3, 2.55, 13.6, 2.20, 8.5}, {10.0, 5.00, 9.4, 5.95, 3.6}}}};
 
-// Modelled times of one kernel; bh heads of T rows.
+// Modelled times of one kernel and its rounds of workgroups; bh heads of T rows.
 inline void split16_times(int kernel, bool pur, int64_t bh, int64_t T, int D, bool causal, int64_t window,
-                          double* tuned, double* split) {
+                          double* tuned, double* split, double* rounds) {
     const int d = D <= 128 ? (D + 31) / 32 - 1 : 4;
     const int dp = d < 4 ? 32 * (d + 1) : 256;
     const SplitCost& c = kSplitCost[pur ? 1 : 0][d][kernel];
@@ -73,8 +73,8 @@ inline void split16_times(int kernel, bool pur, int64_t bh, int64_t T, int D, bo
     const double moved = bytes / (c.bw * 1e6);
     *tuned = c.ta + c.tc * (double)(((int64_t)longest(rows_tuned) + 63) / 64);
     const double slots = dp <= 64 ? 512 : 256;  // two workgroups per CU, or one (LDS)
-    const double rounds = (double)(int64_t)((blocks + slots - 1) / slots);
-    *split = c.sa * (1.0 + 0.7 * (rounds - 1)) + (c.sc * chain > moved ? c.sc * chain : moved);
+    *rounds = (double)(int64_t)((blocks + slots - 1) / slots);
+    *split = c.sa * (1.0 + 0.7 * (*rounds - 1)) + (c.sc * chain > moved ? c.sc * chain : moved);
 }
 
 // The kernels address a (T, D) slice with 32-bit byte offsets, rows up to T + 256.
@@ -104,14 +104,30 @@ constexpr int split_rank(int bid, int grid, bool two_per_cu) {
 constexpr bool split_two_per_cu(int tile_bytes) { return 2 * (tile_bytes + 4 * 1024) <= 160 * 1024; }
 
 // bwd: dQ and dK/dV together (one side's row sums feed the other's kernel).
+//
+// The model takes a block's whole range for its length.  With document ids,
+// whose lengths the host does not know, it may be a fraction of that, and then
+// a split block's start weighs more than its chain.  At most head dims the
+// split kernels stay ahead, or even, from documents of 128 tokens on.  Not so
+// Born's at padded head dim 128, one block per CU with the longest start: the
+// forward is no faster at a mean of 512 tokens and a fifth slower at 128, and
+// the backward loses in launches of more than two rounds of blocks.  Tuned and
+// split, by mean document length:
+//   Born B1 H2 D128 dense        fwd T1000 512: 20.3 / 20.5   T1531 128: 19.2 / 24.0
+//   Born B1 H8 T3000 D128        fwd 128: 19.5 / 35.7   bwd 128: 61.3 / 93.4
+//   Born B1 H8 T1000 D96 dense   fwd 128: 17.9 / 20.7   bwd 128: 48.1 / 42.5
+//   purified B2 H8 T1531 D96     fwd 128: 31.3 / 35.0   512: 66.9 / 40.6
 template <class Args>
 inline bool split16_pays(const Args& a, bool bwd, bool pur) {
     const int64_t bh = (int64_t)a.B * a.H;
     if (!split16_addressable(a.T)) return false;
+    const bool born_docs = a.doc != nullptr && !pur && a.D > 96 && a.D <= 128;
+    if (born_docs && !bwd) return false;
     double tuned = 0, split = 0;
     for (int k = bwd ? kSplitDq : kSplitFwd; k <= (bwd ? kSplitDkdv : kSplitFwd); ++k) {
-        double t, s;
-        split16_times(k, pur, bh, a.T, a.D, a.is_causal != 0, a.window, &t, &s);
+        double t, s, rounds;
+        split16_times(k, pur, bh, a.T, a.D, a.is_causal != 0, a.window, &t, &s, &rounds);
+        if (born_docs && rounds > 2) return false;
         tuned += t;
         split += s;
     }

@@ -72,9 +72,10 @@ def rule(tmp_path_factory):
 @pytest.mark.parametrize("case", HEAD_DIMS, ids=str)
 def test_every_head_dim_and_mask_takes_the_split_kernels(rule, case):
     """All four passes, but the Born forward at padded head dims 96 and 128
-    with a window (too few tiles a block at this length)."""
+    with a window (too few tiles a block at this length) and at 128 with
+    documents."""
     B, H, T, D, mask = case
-    born_fwd = D <= 64 or D > 128 or not MASKS[mask][1]
+    born_fwd = D <= 64 or D > 128 or mask in ("causal", "dense") or (D <= 96 and mask in ("docs", "docs_dense"))
     assert rule(*case) == [born_fwd, True, True, True]
 
 
@@ -93,6 +94,13 @@ def test_full_chip_of_purified_blocks(rule):
                                      (4096, 4096, 4, 64), (1, 1, 1 << 28, 256)])
 def test_others_keep_the_tuned_kernels(rule, B, H, T, D):
     assert not any(rule(B, H, T, D))
+
+
+# Born launches with documents that measured faster on the tuned kernels.
+@pytest.mark.parametrize("case,which", [((1, 8, 3000, 128, "docs"), 0), ((1, 8, 3000, 128, "docs"), 1),
+                                        ((1, 2, 1531, 128, "docs_dense"), 0), ((1, 4, 3000, 120, "docs"), 0)])
+def test_measured_slower_keep_the_tuned_kernels(rule, case, which):
+    assert not rule(*case)[which]
 
 
 OFFSETS = """
