@@ -711,7 +711,7 @@ inline int f32_groups(int B, int H, int T) { return (int)f32_blocks((int64_t)B *
 template <bool PUR, class Args>
 hipError_t launch_f32_fwd(const Args& a, hipStream_t st) {
     const dim3 grid((unsigned)f32_groups(a.B, a.H, a.T));
-    const int nw = f32_waves((int64_t)a.B * a.H, a.T, a.D, a.is_causal != 0, a.window);
+    const int nw = f32_waves((int64_t)a.B * a.H, a.T, a.D, a.is_causal != 0, a.window, a.doc != nullptr);
     QDL_F32_DP(a.D, {
         QDL_F32_NW(nw, {
             hipLaunchKernelGGL((born_f32_fwd_kernel<DPV, PUR, NWV>), grid, dim3(64 * NWV), 0, st, a);
@@ -724,7 +724,7 @@ hipError_t launch_f32_fwd(const Args& a, hipStream_t st) {
 template <bool PUR, class Args>
 hipError_t launch_f32_bwd(const Args& a, hipStream_t st) {
     const dim3 grid((unsigned)f32_groups(a.B, a.H, a.T));
-    const int nw = f32_waves((int64_t)a.B * a.H, a.T, a.D, a.is_causal != 0, a.window);
+    const int nw = f32_waves((int64_t)a.B * a.H, a.T, a.D, a.is_causal != 0, a.window, a.doc != nullptr);
     QDL_F32_DP(a.D, {
         QDL_F32_NW(nw, {
             hipLaunchKernelGGL((born_f32_dq_kernel<DPV, PUR, NWV>), grid, dim3(64 * NWV), 0, st, a);

@@ -20,7 +20,7 @@ MAIN = """
 int main(int, char** v) {
     const int64_t BH = atoll(v[1]), T = atoll(v[2]);
     const int D = atoi(v[3]), causal = atoi(v[4]), docs = atoi(v[6]);
-    printf("%%d ", qdl::f32_waves(BH, T, D, causal, atoi(v[5])));
+    printf("%%d ", qdl::f32_waves(BH, T, D, causal, atoi(v[5]), docs));
     for (int pur = 0; pur < 2; ++pur)
         for (int bwd = 0; bwd < 2; ++bwd) printf("%%d ", qdl::f32_staged(pur, bwd, BH, T, D, causal, atoi(v[5]), docs));
 }
@@ -71,3 +71,9 @@ def test_staged_launches(rule, BH, T, D, window, docs, staged):
 ])
 def test_waves_per_block(rule, BH, T, D, causal, window, waves):
     assert rule(BH, T, D, causal, window)[0] == waves
+
+
+@pytest.mark.parametrize("BH,T,D,window,waves", [(64, 512, 128, 384, 4), (18, 1531, 96, 384, 4), (8, 8192, 96, 384, 1),
+                                                 (128, 512, 96, 0, 1)])
+def test_waves_per_block_with_documents(rule, BH, T, D, window, waves):
+    assert rule(BH, T, D, 1, window, 1)[0] == waves
