@@ -191,35 +191,35 @@ def qk_prologue_backward(gq, gk, q_out, k_out, q_rinv, k_rinv, cos=None, sin=Non
                          q_layout=None, k_layout=None):
     """No-autograd backward: input gradients (None where the output gradient
     is None), written with ``(shape, strides)`` layouts (default contiguous)."""
-    B, H, T, D = q_out.shape
-    cos2, sin2 = _prep_tables(cos, sin, D // 2, T, q_out.device)
     jobs = []  # per tensor: (slot, output gradient, output, 1/norm, input gradient)
     for which, (g, out, rinv, layout) in enumerate(((gq, q_out, q_rinv, q_layout), (gk, k_out, k_rinv, k_layout))):
         if g is None:
             continue
         dx = _grad_like(layout or (tuple(out.shape), tuple(out.stride())), out.dtype, out.device)
         jobs.append((which, g.to(out.dtype).contiguous(), out, rinv, dx))
-    # One launch for both, unless their dtypes or devices differ.
-    together = len({(j[2].dtype, j[2].device) for j in jobs}) <= 1
+    # One launch for both, unless their shapes, dtypes or devices differ.
+    together = len({(j[2].shape, j[2].dtype, j[2].device) for j in jobs}) <= 1
     for batch in [jobs] if together and jobs else [[j] for j in jobs]:
-        _launch_bwd(batch, (B, H, T, D), cos2, sin2)
+        _launch_bwd(batch, cos, sin)
     grads = {j[0]: j[4] for j in jobs}
     return grads.get(0), grads.get(1)
 
 
-def _launch_bwd(jobs, shape, cos2, sin2) -> None:
-    """The prologue backward of one or both tensors of one dtype and device."""
+def _launch_bwd(jobs, cos, sin) -> None:
+    """The prologue backward of one or both tensors of one shape, dtype and device."""
     lib = _native.load()
+    out = jobs[0][2]
+    B, H, T, D = out.shape
+    cos2, sin2 = _prep_tables(cos, sin, D // 2, T, out.device)
     gs, ys, rs, ds, strides = [None] * 2, [None] * 2, [None] * 2, [None] * 4, []
-    for which, g, out, rinv, dx in jobs:
+    for which, g, y, rinv, dx in jobs:
         st = _strides(dx)
         strides.append(st)  # alive until the call
-        gs[which], ys[which], rs[which] = g.data_ptr(), out.data_ptr(), rinv.data_ptr()
+        gs[which], ys[which], rs[which] = g.data_ptr(), y.data_ptr(), rinv.data_ptr()
         ds[2 * which], ds[2 * which + 1] = dx.data_ptr(), st.data_ptr()
-    out = jobs[0][2]
     with torch.cuda.device(out.device):
         rc = lib.qdl_flash_born_qk_prologue_bwd(
-            _DTYPE_CODE[out.dtype], *shape, *gs, *ys, *rs,
+            _DTYPE_CODE[out.dtype], B, H, T, D, *gs, *ys, *rs,
             cos2.data_ptr() if cos2 is not None else None,
             sin2.data_ptr() if sin2 is not None else None,
             cos2.shape[1] if cos2 is not None else 0,

@@ -290,3 +290,30 @@ def test_prologue_gradient_layout_rule():
     e = torch.empty(1, 4, 8, 16).expand(2, 4, 8, 16)  # stride 0: overlapping
     assert not _dense_layout(tuple(e.shape), e.stride())
     assert _dense_layout((1, 4, 8, 16), (999, 128, 16, 1))  # size-1 dims are free
+
+
+def test_prologue_backward_of_two_shapes(monkeypatch):
+    """qk_prologue_backward launches a q and a k of different shapes one by one,
+    each with its own: the kernel indexes every tensor by the shape it is given."""
+    import contextlib
+
+    from quantumdlblocks_amd.kernels import qk_prologue as qp
+
+    calls = []
+
+    class Lib:
+        def qdl_flash_born_qk_prologue_bwd(self, *args):
+            calls.append((args[1:5], [x is not None for x in args[5:7]]))
+            return 0
+
+    monkeypatch.setattr(qp._native, "load", Lib)
+    monkeypatch.setattr(qp, "_stream_ptr", lambda device: 0)
+    monkeypatch.setattr(torch.cuda, "device", lambda device: contextlib.nullcontext())
+    q, k = torch.zeros(2, 4, 6, 8), torch.zeros(2, 1, 6, 8)
+    rinv = [x.new_zeros(x.shape[:3]) for x in (q, k)]
+    dq, dk = qp.qk_prologue_backward(q, k, q, k, *rinv)
+    assert (dq.shape, dk.shape) == (q.shape, k.shape)
+    assert calls == [(tuple(q.shape), [True, False]), (tuple(k.shape), [False, True])]
+    calls.clear()
+    qp.qk_prologue_backward(q, q, q, q, rinv[0], rinv[0])
+    assert calls == [(tuple(q.shape), [True, True])]  # one launch for equal ones
