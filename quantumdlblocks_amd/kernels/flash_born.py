@@ -403,7 +403,11 @@ class _FlashPurifiedBornAttentionFn(torch.autograd.Function):
     returned cast to the compute dtype; Z is fp32 with eps.  backward: returns
     dq, dk, dv in the original input dtypes, dscale and dtau in their
     parameters' shapes and dtypes, and None for eps_base, is_causal, eps,
-    window_size, doc_ids.
+    window_size, doc_ids, grad_enabled.
+
+    ``grad_enabled``: the caller's grad mode.  ``apply`` switches it off before
+    ``forward``, and ``ctx.needs_input_grad`` names every input that requires
+    a gradient, also where none is recorded.
     """
 
     @staticmethod
@@ -419,6 +423,7 @@ class _FlashPurifiedBornAttentionFn(torch.autograd.Function):
         eps: float,
         window_size: int = 0,
         doc_ids: torch.Tensor | None = None,
+        grad_enabled: bool = True,
     ) -> torch.Tensor:
         lib = _native.load()
         target = _autocast_dtype(q) or v.dtype
@@ -438,7 +443,8 @@ class _FlashPurifiedBornAttentionFn(torch.autograd.Function):
         # fp32 one only for a backward.
         out = torch.empty((B, H, T, dp), dtype=target, device=dev) if target != torch.float32 else None
         out_f32 = None
-        if out is None or any(ctx.needs_input_grad[:5]):
+        wanted = [grad_enabled and needs for needs in ctx.needs_input_grad[:5]]
+        if out is None or any(wanted):
             out_f32 = torch.empty((B, H, T, dp), dtype=torch.float32, device=dev)
         z = torch.empty((B, H, T), dtype=torch.float32, device=dev)
         window = max(int(window_size), 0)
@@ -448,7 +454,7 @@ class _FlashPurifiedBornAttentionFn(torch.autograd.Function):
             scale_p, n_scale, scale_value, 0 if doc_c is None else doc_c.data_ptr(),
             1 if is_causal else 0, window, float(eps),
             out16=0 if out is None else out.data_ptr(), purified=1, tau=tau_p, n_tau=n_tau, tau_value=tau_value, eps_base=float(eps_base),
-            param_grads=1 if ctx.needs_input_grad[3] or ctx.needs_input_grad[4] else 0))
+            param_grads=1 if wanted[3] or wanted[4] else 0))
         ctx.save_for_backward(q_c, k_c, v_c, out_f32, z, scale_flat, tau_flat, doc_c)
         ctx.is_causal = bool(is_causal)
         ctx.window_size = window
@@ -494,7 +500,7 @@ class _FlashPurifiedBornAttentionFn(torch.autograd.Function):
             dq, dk, dv = dq[..., :D], dk[..., :D], dv[..., :D]
         qd, kd, vd = ctx.dtypes
         params = (None if g is None else g.view(sd[0]).to(sd[1]) for g, sd in zip((dscale, dtau), ctx.shapes))
-        return (dq.to(qd), dk.to(kd), dv.to(vd), *params, None, None, None, None, None)
+        return (dq.to(qd), dk.to(kd), dv.to(vd), *params, None, None, None, None, None, None)
 
 
 def _run_triton_flash_purified_born(
@@ -511,7 +517,8 @@ def _run_triton_flash_purified_born(
 ) -> torch.Tensor:
     """Direct entry to the GPU kernels (reference name, flash_born.py:1273-1287)."""
     return _apply(
-        _FlashPurifiedBornAttentionFn, q, k, v, scale_t, tau_t, eps_base, is_causal, eps, int(window_size), doc_ids
+        _FlashPurifiedBornAttentionFn, q, k, v, scale_t, tau_t, eps_base, is_causal, eps, int(window_size), doc_ids,
+        torch.is_grad_enabled(),
     )
 
 

@@ -294,15 +294,16 @@ def fused_qk_rope_l2_normalize(
 
 class _BornQKPrologueFn(torch.autograd.Function):
     """Forward: Born attention of (q', k', v) with q' = l2_normalize(rope(q)),
-    k' likewise, in one call of ``qdl_flash_born_fwd_qk_prologue`` (for bf16,
-    D = 64, no documents or window: the prologue kernel on K alone, then one
-    attention kernel that normalises each query block as it loads it).  Saves
-    q', k' and 1/norm when a gradient is needed (otherwise 1/norm and q' are
-    not written).  Backward: the attention backward on (q', k', v), then the
+    k' likewise, in one library call (for bf16, D = 64, dense or causal, with
+    documents also under a causal window, and blocks enough for the tuned
+    kernels: the prologue kernel on K alone, then one attention kernel that
+    normalises each query block as it loads it).  Saves q', k' and 1/norm when
+    a gradient is needed (``grad_enabled``, the caller's grad mode, and an
+    input that requires one; otherwise 1/norm and q' are not written).  Backward: the attention backward on (q', k', v), then the
     prologue backward into q and k (their dtypes and strides)."""
 
     @staticmethod
-    def forward(ctx, q, k, v, scale, cos, sin, is_causal, eps, window_size, doc_ids, norm_eps):
+    def forward(ctx, q, k, v, scale, cos, sin, is_causal, eps, window_size, doc_ids, norm_eps, grad_enabled=True):
         from .flash_born import _aligned, _autocast_dtype, _check_inputs, _parameter, _run_call
 
         lib = _native.load()
@@ -322,7 +323,7 @@ class _BornQKPrologueFn(torch.autograd.Function):
         z = torch.empty((B, H, T), dtype=torch.float32, device=dev)
         q_out = torch.empty_like(out)
         k_out = torch.empty_like(out)
-        grad = any(ctx.needs_input_grad[:4])
+        grad = grad_enabled and any(ctx.needs_input_grad[:4])
         q_r = torch.empty_like(z) if grad else None
         k_r = torch.empty_like(z) if grad else None
         window = max(int(window_size), 0)
@@ -378,7 +379,7 @@ class _BornQKPrologueFn(torch.autograd.Function):
         qd, kd, vd = ctx.dtypes
         return (dq.to(qd), dk.to(kd), dv.to(vd),
                 None if dscale is None else dscale.view(ctx.scale_shape).to(ctx.scale_dtype),
-                None, None, None, None, None, None, None)
+                None, None, None, None, None, None, None, None)
 
 
 def flash_born_attention_qk_prologue(
@@ -403,9 +404,10 @@ def flash_born_attention_qk_prologue(
     ``(B, T, H, D)`` projection output viewed as ``(B, H, T, D)``); v: any
     ``(B, H, T, D)``; cos, sin as for ``fused_qk_rope_l2_normalize`` (or None:
     normalisation only); the other arguments as for ``flash_born_attention``.
-    On the GPU, bf16 with D = 64 and no documents or window runs as one
-    kernel; other cases run the prologue kernel and then the attention
-    kernels.  CPU tensors take the reference's eager formulation of both.
+    On the GPU, bf16 with D = 64 (dense or causal; with documents also under a
+    causal window) normalises Q in the attention kernel's loads, but for
+    launches of few blocks; other cases run the prologue kernel and then the
+    attention kernels.  CPU tensors take the reference's eager formulation of both.
     """
     from .flash_born import MAX_HEAD_DIM, flash_born_attention
 
@@ -418,4 +420,4 @@ def flash_born_attention_qk_prologue(
         qn, kn = fused_qk_rope_l2_normalize(q, k, cos, sin, norm_eps)
         return flash_born_attention(qn, kn, v, scale, is_causal, eps, window_size, doc_ids)
     return _BornQKPrologueFn.apply(q, k, v, scale, cos, sin, bool(is_causal), float(eps), int(window_size),
-                                   doc_ids, float(norm_eps))
+                                   doc_ids, float(norm_eps), torch.is_grad_enabled())

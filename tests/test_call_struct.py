@@ -140,3 +140,65 @@ def test_purified_output_in_the_compute_dtype(cuda_device, dtype, D, T, mask):
     assert plain.dtype == out.dtype == dtype and out.is_contiguous()
     assert torch.equal(plain, out)
     assert torch.equal(out, kept.to(dtype)[..., :D])
+
+
+def _field(block, name):
+    """One field of a packed block, by its name in the C struct."""
+    body = re.search(r"typedef struct qdl_born_call \{(.*?)\} qdl_born_call;", open(HEADER).read(), re.S).group(1)
+    at = 0
+    for decl in re.sub(r"/\*.*?\*/", "", body, flags=re.S).split(";"):
+        for field in decl.split(",") if decl.strip() else []:
+            word, n = re.search(r"(\w+)\s*(?:\[(\d+)\])?\s*$", field).groups()
+            if word == name:
+                return int.from_bytes(block[8 * at:8 * at + 8], "little")
+            at += int(n or 1)
+    raise KeyError(name)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("mode", ["grad", "no_grad", "inference_mode"])
+def test_trained_parameters_without_a_backward(monkeypatch, mode, dtype):
+    """What a purified call keeps for its backward is asked for where one can
+    follow, not wherever a parameter requires a gradient."""
+    from quantumdlblocks_amd.kernels import flash_born as fb
+
+    blocks = []
+    monkeypatch.setattr(fb, "_run_call", lambda fn, what, device, block: blocks.append(block))
+    q = torch.zeros(1, 2, 8, 16, dtype=dtype)
+    scale, tau = (torch.full((2,), x, requires_grad=True) for x in (8.0, 0.0625))
+    grad_mode = {"grad": torch.enable_grad, "no_grad": torch.no_grad, "inference_mode": torch.inference_mode}[mode]
+    with grad_mode():
+        out = fb._run_triton_flash_purified_born(q, q, q, scale, tau, 0.05, True, 1e-8)
+    assert out.requires_grad == (mode == "grad")
+    assert (_field(blocks[0], "out") != 0, _field(blocks[0], "param_grads")) == (mode == "grad", mode == "grad")
+    assert _field(blocks[0], "out16") != 0
+
+
+@pytest.mark.parametrize("grad_enabled", [True, False])
+def test_trained_scale_of_the_prologue_without_a_backward(monkeypatch, grad_enabled):
+    from quantumdlblocks_amd.kernels import flash_born as fb
+    from quantumdlblocks_amd.kernels.qk_prologue import _BornQKPrologueFn
+
+    blocks = []
+    monkeypatch.setattr(fb, "_run_call", lambda fn, what, device, block: blocks.append(block))
+    q = torch.zeros(1, 2, 8, 16, dtype=torch.bfloat16)
+    _BornQKPrologueFn.apply(q, q, q, torch.ones(2, requires_grad=True), None, None, True, 1e-12, 0, None, 1e-12,
+                            grad_enabled)
+    assert (_field(blocks[0], "q_rinv") != 0) == (_field(blocks[0], "k_rinv") != 0) == grad_enabled
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32], ids=str)
+def test_trained_parameters_under_no_grad_on_the_gpu(cuda_device, dtype):
+    """The same call as one with plain numbers, bitwise, and gradients as
+    before where they are recorded."""
+    from quantumdlblocks_amd import flash_purified_born_attention
+
+    g = torch.Generator("cpu").manual_seed(0)
+    q, k, v = (torch.randn(1, 2, 1000, 64, generator=g).mul(0.3).to(cuda_device, dtype) for _ in range(3))
+    scale, tau = (torch.tensor(x, device=cuda_device, requires_grad=True) for x in (2.0, 0.02))
+    with torch.no_grad():
+        assert torch.equal(flash_purified_born_attention(q, k, v, scale, tau),
+                           flash_purified_born_attention(q, k, v, 2.0, 0.02))
+    flash_purified_born_attention(q, k, v, scale, tau).float().square().mean().backward()
+    assert torch.isfinite(scale.grad).all() and torch.isfinite(tau.grad).all()
