@@ -37,8 +37,8 @@ inline int f32_waves(int64_t BH, int64_t T, int D, bool causal, int64_t window, 
 }
 
 // Launches up to D = 128 that the staged kernels keep: without causality and
-// with at least 256 whole blocks of their 128 rows (512 with a window, whose
-// blocks differ in length), at padded head dim 128, and the Born forward at 96 too.
+// with at least 256 blocks of their 128 rows (512 with a window, whose blocks
+// differ in length; none at T below 128), at padded head dim 128, and the Born forward at 96 too.
 // There the chip is full with either, and the four waves of a staged block
 // read one tile where a wave-split wave reads its own.  With documents only
 // the purified backward (the Born forward does not screen their ranges; the
@@ -49,7 +49,7 @@ inline int f32_waves(int64_t BH, int64_t T, int D, bool causal, int64_t window, 
 inline bool f32_staged(bool purified, bool backward, int64_t BH, int64_t T, int D, bool causal, int64_t window,
                        bool documents) {
     if (D > kF32MaxD) return true;
-    if (causal || T / 128 * BH < (window > 0 ? 512 : 256)) return false;
+    if (causal || T < 128 || (T + 127) / 128 * BH < (window > 0 ? 512 : 256)) return false;
     if (documents) return purified && backward && D > 96;
     return D > (purified || backward ? 96 : 64);
 }

@@ -47,14 +47,15 @@ def rule(tmp_path_factory):
 
 @pytest.mark.parametrize("BH,T,D,window,docs,staged", [
     (256, 512, 128, 0, 0, [1, 1, 1, 1]),   # full chips: both passes, Born and purified
-    (80, 1000, 104, 256, 0, [1, 1, 1, 1]),
+    (32, 1000, 128, 0, 0, [1, 1, 1, 1]),
+    (64, 1000, 104, 256, 0, [1, 1, 1, 1]),
     (128, 512, 96, 0, 0, [1, 0, 0, 0]),
     (128, 512, 72, 256, 0, [1, 0, 0, 0]),
     (128, 512, 128, 0, 1, [0, 0, 0, 1]),
     (128, 512, 96, 0, 1, [0, 0, 0, 0]),
     (128, 512, 64, 0, 0, [0, 0, 0, 0]),
     (255, 128, 128, 0, 0, [0, 0, 0, 0]),   # too few blocks of 128 rows
-    (512, 100, 128, 0, 0, [0, 0, 0, 0]),   # none of them whole
+    (512, 100, 128, 0, 0, [0, 0, 0, 0]),   # none of them full
     (4, 8192, 128, 256, 0, [0, 0, 0, 0]),  # enough, but of unequal length
     (1, 64, 136, 0, 1, [1, 1, 1, 1]),      # wider heads: always
 ])
