@@ -104,7 +104,8 @@ def get_rdna4_autotune_configs() -> list[dict[str, int]]:
 def get_mi355x_launch_meta(head_dim: int = 64, dtype: torch.dtype = torch.bfloat16) -> dict[str, int]:
     """Tiling of the gfx950 forward kernels for this head dim and dtype: the
     tuned 16-bit kernels' (launches of few blocks take 32- or 64-row blocks)
-    and the staged fp32 kernels' (fp32 up to head dim 128 takes 32-row blocks)."""
+    and the staged fp32 kernels' (most fp32 launches up to head dim 128 take
+    32-row blocks)."""
     dp = (max(8, head_dim) + 31) // 32 * 32
     if dtype == torch.float32:
         return {"BLOCK_M": 128, "BLOCK_N": 32, "waves": 4, "queries_per_wave": 32,
